@@ -4,8 +4,7 @@
 // Feedback kernels: the reference recomputes sum(logits^2) in every thread
 // (O(rows * cols)); here each 1024-thread workgroup reduces it once with wave64
 // shuffles and then writes 1024 outputs, so the cost is O(rows * cols / 1024).
-#include <cfloat>
-
+#include "argmax.cuh"
 #include "common.h"
 #include "internal.h"
 #include "rtxllm/decode_kernels.h"
@@ -97,58 +96,27 @@ hipError_t launch_feedback(const float* logits, const float* gate, float* cache,
 
 // ---- argmax ---------------------------------------------------------------
 
-__device__ __forceinline__ bool better(float v, std::uint32_t i, float bv, std::uint32_t bi) {
-  return v > bv || (v == bv && i < bi);
-}
-
-// One workgroup; each thread scans a strided slice keeping the first maximum,
-// then a wave64 + LDS tournament keeps the lowest index among equal maxima.
-// Initial (value, index) = (-FLT_MAX, 0) as in the reference, so NaNs never win.
-__global__ __launch_bounds__(1024) void argmax_token_kernel(const float* __restrict__ logits, std::uint32_t* token,
-                                                             std::uint32_t rows, int mode, std::uint32_t vocab,
-                                                             std::uint32_t offset) {
-  __shared__ float sv[16];
-  __shared__ std::uint32_t si[16];
-  float bv = -FLT_MAX;
-  std::uint32_t bi = 0u;
-  for (std::uint32_t r = threadIdx.x; r < rows; r += blockDim.x) {
-    const float v = logits[r];
-    if (better(v, r, bv, bi)) {
-      bv = v;
-      bi = r;
-    }
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o, 64);
-    const std::uint32_t oi = __shfl_xor(bi, o, 64);
-    if (better(ov, oi, bv, bi)) {
-      bv = ov;
-      bi = oi;
-    }
-  }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0) {
-    sv[wave] = bv;
-    si[wave] = bi;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const int nw = blockDim.x >> 6;
-    for (int i = 1; i < nw; ++i)
-      if (better(sv[i], si[i], bv, bi)) {
-        bv = sv[i];
-        bi = si[i];
-      }
-    token[0] = mode == 0 ? (bi + token[0] + 1u) % 32000u : (bi + offset) % vocab;
-  }
+// One workgroup per call (argmax.cuh: why, and the rules for ties and NaN).
+template <std::uint32_t U>
+__global__ __launch_bounds__(kArgmaxThreads) void argmax_token_kernel(const float* __restrict__ logits,
+                                                                      std::uint32_t* token, std::uint32_t rows,
+                                                                      int mode, std::uint32_t vocab,
+                                                                      std::uint32_t offset) {
+  const std::uint32_t before = (threadIdx.x == 0u && mode == 0) ? token[0] : 0u;  // read ahead of the scan
+  const std::uint32_t bi = argmax_row<U>(logits, rows);
+  if (threadIdx.x == 0u) token[0] = mode == 0 ? (bi + before + 1u) % 32000u : (bi + offset) % vocab;
 }
 
 }  // namespace
 
 hipError_t launch_argmax_token(const float* logits, std::uint32_t* token, std::uint32_t rows, int mode,
                                std::uint32_t vocab, std::uint32_t offset, hipStream_t stream) {
-  hipLaunchKernelGGL(argmax_token_kernel, dim3(1), dim3(1024), 0, stream, logits, token, rows, mode, vocab, offset);
+  if (rows <= kArgmaxShort)
+    hipLaunchKernelGGL(argmax_token_kernel<2>, dim3(1), dim3(kArgmaxThreads), 0, stream, logits, token, rows, mode,
+                       vocab, offset);
+  else
+    hipLaunchKernelGGL(argmax_token_kernel<8>, dim3(1), dim3(kArgmaxThreads), 0, stream, logits, token, rows, mode,
+                       vocab, offset);
   return hipGetLastError();
 }
 

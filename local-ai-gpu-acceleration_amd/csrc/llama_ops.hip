@@ -15,8 +15,7 @@
 // (decode_kernels.cu:327-343) at angle pos * theta^(-2i/d), silu(v) = v / (1 +
 // exp(-v)) (main.cpp:1435-1503), Q5_K dequant (main.cpp:1231-1259), argmax with
 // the lowest index among maxima (decode_kernels.cu:2993-3031).
-#include <cfloat>
-
+#include "argmax.cuh"
 #include "dequant.cuh"
 #include "layer.h"
 #include "layer_common.cuh"
@@ -117,33 +116,12 @@ __global__ __launch_bounds__(kOpThreads) void q16_stage_kernel(const float* __re
   q16[static_cast<std::size_t>(r) * slots + idx] = v;
 }
 
-// One workgroup per vector: the reference's argmax scan (start (-FLT_MAX, 0),
-// strictly greater wins, equal values keep the lower index; NaN never wins).
-__global__ __launch_bounds__(1024) void argmax_rows_kernel(const float* __restrict__ x, std::uint32_t n,
-                                                           std::uint32_t* __restrict__ index) {
-  __shared__ float sv[16];
-  __shared__ std::uint32_t si[16];
-  auto better = [](float v, std::uint32_t i, float bv, std::uint32_t bi) { return v > bv || (v == bv && i < bi); };
-  const float* row = x + static_cast<std::size_t>(blockIdx.x) * n;
-  float bv = -FLT_MAX;
-  std::uint32_t bi = 0u;
-  for (std::uint32_t r = threadIdx.x; r < n; r += blockDim.x) {
-    const float v = row[r];
-    if (better(v, r, bv, bi)) bv = v, bi = r;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o, 64);
-    const std::uint32_t oi = __shfl_xor(bi, o, 64);
-    if (better(ov, oi, bv, bi)) bv = ov, bi = oi;
-  }
-  const std::uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-  if (lane == 0u) sv[wave] = bv, si[wave] = bi;
-  __syncthreads();
-  if (threadIdx.x != 0u) return;
-  for (std::uint32_t w = 1; w < blockDim.x / 64u; ++w)
-    if (better(sv[w], si[w], bv, bi)) bv = sv[w], bi = si[w];
-  index[blockIdx.x] = bi;
+// One workgroup per vector (argmax.cuh).
+template <std::uint32_t U>
+__global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(const float* __restrict__ x, std::uint32_t n,
+                                                                     std::uint32_t* __restrict__ index) {
+  const std::uint32_t i = argmax_row<U>(x + static_cast<std::size_t>(blockIdx.x) * n, n);
+  if (threadIdx.x == 0u) index[blockIdx.x] = i;
 }
 
 bool group_ok(std::uint32_t n_heads, std::uint32_t n_kv) {
@@ -243,6 +221,9 @@ extern "C" hipError_t rtxllm_argmax(const float* x, uint32_t n, uint32_t count, 
                                     hipStream_t stream) {
   if (x == nullptr || index == nullptr || n == 0u || count == 0u || count > 65535u * 1024u)
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(argmax_rows_kernel, dim3(count), dim3(1024), 0, stream, x, n, index);
+  if (n <= kArgmaxShort)
+    hipLaunchKernelGGL(argmax_rows_kernel<2>, dim3(count), dim3(kArgmaxThreads), 0, stream, x, n, index);
+  else
+    hipLaunchKernelGGL(argmax_rows_kernel<8>, dim3(count), dim3(kArgmaxThreads), 0, stream, x, n, index);
   return hipGetLastError();
 }
