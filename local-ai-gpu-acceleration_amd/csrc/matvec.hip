@@ -41,17 +41,41 @@ bool pointers_ok(int fmt, const void* payload, const void* meta, const void* x, 
 // ---- bit-exact dequant -----------------------------------------------------
 
 
-// One workgroup of 256 threads per block; thread v writes value v.
+// Four fp32 outputs stored at once; the caller's buffer may have any 4-byte
+// alignment (gfx950 stores unaligned 16-byte vectors).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
+// A wave expands kDequantBlocks consecutive blocks (out is the blocks in order:
+// 256 values each), lane l four values of each: 1 KB of whole lines per store.
+// The kernel is bound by its writes (fp32 out is 7 to 12 times the pack's
+// bytes): nontemporal, as nothing here reads them again. Q4_K 14336 x 4096:
+// 38.5 us, 6.95 TB/s of pack and output; one value per thread (the head decoded
+// 256 times a block, 4-byte stores) took 160.0 us.
+constexpr std::uint32_t kDequantBlocks = 4;
 template <int FMT>
 __global__ __launch_bounds__(256) void dequant_kernel(const std::uint8_t* __restrict__ payload,
-                                                      const std::uint8_t* __restrict__ meta, std::uint32_t cols,
+                                                      const std::uint8_t* __restrict__ meta, std::size_t blocks,
                                                       float* __restrict__ out) {
-  const std::size_t blk = blockIdx.x;
-  const std::uint32_t bpr = cols >> 8;
-  const std::size_t row = blk / bpr, b = blk % bpr;
-  const std::uint8_t* p = payload + blk * rtxllm_format_payload_bytes(FMT);
-  const std::uint8_t* m = meta ? meta + blk * rtxllm_format_meta_bytes(FMT) : nullptr;
-  out[row * cols + b * 256u + threadIdx.x] = dequant_value<FMT>(p, m, threadIdx.x);
+  const std::uint32_t lane = threadIdx.x & 63u;
+  const std::size_t b0 = (static_cast<std::size_t>(blockIdx.x) * 4u + (threadIdx.x >> 6)) * kDequantBlocks;
+  auto load = [&](std::size_t b) {
+    return run4_load<FMT>(payload + b * rtxllm_format_payload_bytes(FMT),
+                          meta != nullptr ? meta + b * rtxllm_format_meta_bytes(FMT) : nullptr, lane);
+  };
+  auto store = [&](std::size_t b, const float4& v) {
+    const f32x4_any o = {v.x, v.y, v.z, v.w};
+    __builtin_nontemporal_store(o, reinterpret_cast<f32x4_any*>(out + b * 256u + 4u * lane));
+  };
+  if (b0 + kDequantBlocks <= blocks) {
+    Run4 r[kDequantBlocks];
+#pragma unroll
+    for (std::uint32_t j = 0; j < kDequantBlocks; ++j) r[j] = load(b0 + j);
+    __builtin_amdgcn_sched_barrier(0);  // every block's loads ahead of the first's arithmetic
+#pragma unroll
+    for (std::uint32_t j = 0; j < kDequantBlocks; ++j) store(b0 + j, run4_values<FMT>(r[j], lane));
+  } else {
+    for (std::size_t b = b0; b < blocks; ++b) store(b, run4_values<FMT>(load(b), lane));
+  }
 }
 
 // Unit layouts: the workgroup gathers its block's bytes back into the GGUF
@@ -103,8 +127,9 @@ template <int FMT>
 hipError_t launch_dequant_fmt(const std::uint8_t* payload, const std::uint8_t* meta, std::uint32_t rows,
                               std::uint32_t cols, float* out, hipStream_t stream) {
   const std::size_t blocks = static_cast<std::size_t>(rows) * (cols / 256u);
-  hipLaunchKernelGGL(dequant_kernel<FMT>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, stream, payload,
-                     meta, cols, out);
+  constexpr std::size_t kPer = 4u * kDequantBlocks;  // blocks per workgroup
+  hipLaunchKernelGGL(dequant_kernel<FMT>, dim3(static_cast<unsigned>((blocks + kPer - 1u) / kPer)), dim3(256), 0,
+                     stream, payload, meta, blocks, out);
   return hipGetLastError();
 }
 

@@ -8,6 +8,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+from rtxllm_amd import formats as F  # noqa: E402
 from rtxllm_amd import ops, packs  # noqa: E402
 from rtxllm_amd._lib import lib  # noqa: E402
 
@@ -58,3 +59,25 @@ def test_argmax_edges(orc, n, offset):
     tok = torch.full((1,), 7, dtype=torch.int32, device="cuda:0")
     assert lib().rtxllm_launch_output_token_sample(xd.data_ptr() + 4 * n, P(tok), n, 50000, 11, ops.stream()) == 0
     assert int(tok.cpu()[0]) == (orc.argmax(x[1]) + 11) % 50000
+
+
+@pytest.mark.parametrize("fmt", sorted(F.PAYLOAD_BYTES), ids=lambda f: F.NAMES[f])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (3, 256), (5, 768), (7, 2304), (33, 4096)])
+def test_dequant_edges_bit_exact(orc, fmt, rows, cols):
+    """Block counts around the kernel's 4 blocks a wave and 16 a workgroup, and an
+    output buffer off its 16-byte alignment; nothing past the end is written."""
+    pack = packs.make_pack(fmt, rows, cols, seed=900 + fmt)
+    d = ops.DevicePack(pack)
+    n = rows * cols
+    big = torch.full((n + 9,), 7.0, dtype=torch.float32, device="cuda:0")
+    src = {F.IQ2S_UNITS: (F.IQ2S, packs.iq2s_from_units), F.IQ3S_UNITS: (F.IQ3S, packs.iq3s_from_units),
+           F.Q4K_RAW_PREDECODED: (F.Q4K_RAW, lambda raw: raw)}.get(fmt)  # its pairs are d sc and dmin m, rounded once
+    ofmt, payload = (fmt, pack.payload) if src is None else (src[0], src[1](pack.payload))
+    ref = orc.dequant(ofmt, payload, pack.meta, rows, cols).reshape(-1)
+    for off in (0, 1):
+        big.fill_(7.0)
+        assert lib().rtxllm_dequant_f32(fmt, P(d.payload), P(d.meta), rows, cols, big.data_ptr() + 4 * off,
+                                        ops.stream()) == 0
+        got = big.cpu().numpy()
+        assert np.array_equal(got[off:off + n].view(np.uint32), ref.view(np.uint32)), off
+        assert np.all(got[:off] == 7.0) and np.all(got[off + n:] == 7.0)
