@@ -36,7 +36,48 @@ __device__ float block_sum256(float v, float* sh) {
   return s;
 }
 
-// One workgroup per vector r of x [count][n].
+// One workgroup of T threads per vector r of x [count][n], the vector held in
+// registers: V 16-byte loads a thread (n <= 4 T V), so it is read once, and the
+// weights are read ahead of the reduction. x, w and out 16-byte aligned, n % 4
+// == 0; in place allowed (a thread writes what it alone read). Against the
+// scalar two-pass kernel below (16 dependent loads, twice): one vector of 4096
+// 8.4 -> 2.4 us, 256 of them 11.5 -> 3.5 us.
+template <std::uint32_t T, std::uint32_t V>
+__global__ __launch_bounds__(T) void rmsnorm_w_vec_kernel(const float* x, const float* __restrict__ w, std::uint32_t n,
+                                                          float eps, float* out) {
+  __shared__ float sh[T / 64u];
+  const std::uint32_t n4 = n / 4u;
+  const std::size_t base = static_cast<std::size_t>(blockIdx.x) * n4;
+  float4 v[V], wv[V];
+#pragma unroll
+  for (std::uint32_t j = 0; j < V; ++j) {
+    const std::uint32_t i = threadIdx.x + T * j, c = i < n4 ? i : n4 - 1u;  // past the end: read again, not summed
+    v[j] = reinterpret_cast<const float4*>(x)[base + c];
+    wv[j] = w != nullptr ? reinterpret_cast<const float4*>(w)[c] : make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+  }
+  float s = 0.0f;
+#pragma unroll
+  for (std::uint32_t j = 0; j < V; ++j) {
+    const float t = fmaf(v[j].w, v[j].w, fmaf(v[j].z, v[j].z, fmaf(v[j].y, v[j].y, v[j].x * v[j].x)));
+    s += threadIdx.x + T * j < n4 ? t : 0.0f;
+  }
+  s = wave_sum(s);
+  if ((threadIdx.x & 63u) == 0u) sh[threadIdx.x >> 6] = s;
+  __syncthreads();
+  float total = sh[0];
+#pragma unroll
+  for (std::uint32_t k = 1; k < T / 64u; ++k) total += sh[k];
+  const float inv = 1.0f / sqrtf(total / static_cast<float>(n) + eps);
+#pragma unroll
+  for (std::uint32_t j = 0; j < V; ++j) {
+    const std::uint32_t i = threadIdx.x + T * j;
+    if (i < n4)  // times 1 without a weight: exact
+      reinterpret_cast<float4*>(out)[base + i] = make_float4(v[j].x * inv * wv[j].x, v[j].y * inv * wv[j].y,
+                                                             v[j].z * inv * wv[j].z, v[j].w * inv * wv[j].w);
+  }
+}
+
+// The rest: unaligned pointers, n % 4 != 0, vectors over 16384 values.
 __global__ __launch_bounds__(kOpThreads) void rmsnorm_w_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                std::uint32_t n, float eps, float* __restrict__ out) {
   __shared__ float sh[kOpThreads / 64];
@@ -141,7 +182,22 @@ extern "C" hipError_t rtxllm_rmsnorm_w(const float* x, const float* weight, uint
                                        float* out, hipStream_t stream) {
   if (x == nullptr || out == nullptr || n == 0u || count == 0u || count > 65535u * 1024u || !(eps >= 0.0f))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(rmsnorm_w_kernel, dim3(count), dim3(kOpThreads), 0, stream, x, weight, n, eps, out);
+  const bool vec = (n % 4u) == 0u && n <= 16384u &&
+                   ((reinterpret_cast<std::uintptr_t>(x) | reinterpret_cast<std::uintptr_t>(weight) |
+                     reinterpret_cast<std::uintptr_t>(out)) % 16u) == 0u;
+  // Few vectors leave the chip idle and the one workgroup's latency is the time:
+  // 16 waves share a vector, one or a few loads each. From half a workgroup per
+  // CU on, four waves a vector keep more of them resident.
+  if (!vec)
+    hipLaunchKernelGGL(rmsnorm_w_kernel, dim3(count), dim3(kOpThreads), 0, stream, x, weight, n, eps, out);
+  else if (n <= 1024u)
+    hipLaunchKernelGGL((rmsnorm_w_vec_kernel<256, 1>), dim3(count), dim3(256), 0, stream, x, weight, n, eps, out);
+  else if (n <= 4096u && count >= 128u)
+    hipLaunchKernelGGL((rmsnorm_w_vec_kernel<256, 4>), dim3(count), dim3(256), 0, stream, x, weight, n, eps, out);
+  else if (n <= 4096u)
+    hipLaunchKernelGGL((rmsnorm_w_vec_kernel<1024, 1>), dim3(count), dim3(1024), 0, stream, x, weight, n, eps, out);
+  else
+    hipLaunchKernelGGL((rmsnorm_w_vec_kernel<1024, 4>), dim3(count), dim3(1024), 0, stream, x, weight, n, eps, out);
   return hipGetLastError();
 }
 
