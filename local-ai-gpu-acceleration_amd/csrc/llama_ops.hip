@@ -154,20 +154,28 @@ __global__ __launch_bounds__(kOpThreads) void silu_mul_kernel(const float* __res
   if (i < n) out[i] = silu(gate[i]) * up[i];
 }
 
-// Workgroup (block b of the row, token t): 256 threads, one value each.
+// Workgroup (four blocks of the row, token t): a wave expands one block, four
+// values a lane (dequant.cuh), and stores 16 bytes a lane at any 4-byte
+// alignment of out. The time is two dependent reads (token, block); against
+// a value a thread, each decoding the head, one row of 4096 4.7 -> 1.9 us, 256
+// rows 5.1 -> 3.2 us.
 __global__ __launch_bounds__(256) void embed_gather_q5k_kernel(const std::uint8_t* __restrict__ table,
                                                                std::uint32_t vocab, std::uint32_t cols,
                                                                const std::uint32_t* __restrict__ tokens,
                                                                float* __restrict__ out) {
-  const std::uint32_t b = blockIdx.x, t = blockIdx.y, bpr = cols / 256u;
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  const std::uint32_t b = 4u * blockIdx.x + (threadIdx.x >> 6), t = blockIdx.y, bpr = cols / 256u;
+  const std::uint32_t lane = threadIdx.x & 63u;
+  if (b >= bpr) return;
   const std::uint32_t tok = tokens[t];
-  float* o = out + static_cast<std::size_t>(t) * cols + 256u * b + threadIdx.x;
-  if (tok >= vocab) {  // no such row: a loud NaN row instead of a silent clamp
-    *o = __builtin_nanf("");
-    return;
+  const float nan = __builtin_nanf("");
+  f32x4_any v = {nan, nan, nan, nan};  // no such row: a loud NaN row instead of a silent clamp
+  if (tok < vocab) {
+    const std::uint8_t* blk = table + (static_cast<std::size_t>(tok) * bpr + b) * 176u;
+    const float4 x = run4_values<RTXLLM_FMT_Q5K>(run4_load<RTXLLM_FMT_Q5K>(blk, nullptr, lane), lane);
+    v = f32x4_any{x.x, x.y, x.z, x.w};
   }
-  const std::uint8_t* blk = table + (static_cast<std::size_t>(tok) * bpr + b) * 176u;
-  *o = dequant_value<RTXLLM_FMT_Q5K>(blk, nullptr, threadIdx.x);
+  *reinterpret_cast<f32x4_any*>(out + static_cast<std::size_t>(t) * cols + 256u * b + 4u * lane) = v;
 }
 
 // fp32 queries q [count][n_heads][128] -> the attention's query operand (q16):
@@ -274,7 +282,7 @@ extern "C" hipError_t rtxllm_embed_gather_q5k(const uint8_t* table, uint32_t voc
   if (table == nullptr || tokens == nullptr || out == nullptr || vocab == 0u || cols == 0u || (cols % 256u) != 0u ||
       count == 0u || count > 65535u || (reinterpret_cast<std::uintptr_t>(table) % 4u) != 0u)
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(embed_gather_q5k_kernel, dim3(cols / 256u, count), dim3(256), 0, stream, table, vocab, cols,
+  hipLaunchKernelGGL(embed_gather_q5k_kernel, dim3((cols / 256u + 3u) / 4u, count), dim3(256), 0, stream, table, vocab, cols,
                      tokens, out);
   return hipGetLastError();
 }
