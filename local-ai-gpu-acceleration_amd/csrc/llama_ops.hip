@@ -154,6 +154,23 @@ __global__ __launch_bounds__(kOpThreads) void silu_mul_kernel(const float* __res
   if (i < n) out[i] = silu(gate[i]) * up[i];
 }
 
+// Four values a thread where the three pointers are 16-byte aligned; the last
+// n % 4 values one each by the first threads past the vectors. 14336 values 4.6 -> 2.1 us
+// against one value a thread; 256 x 14336 9.0 -> 8.0 us (44 MB: 5.5 TB/s, at the
+// copy rate).
+__global__ __launch_bounds__(kOpThreads) void silu_mul_vec_kernel(const float* gate, const float* up, std::size_t n,
+                                                                  float* out) {
+  const std::size_t i = static_cast<std::size_t>(blockIdx.x) * kOpThreads + threadIdx.x, n4 = n / 4u;
+  if (i < n4) {
+    const float4 g = reinterpret_cast<const float4*>(gate)[i], u = reinterpret_cast<const float4*>(up)[i];
+    reinterpret_cast<float4*>(out)[i] =
+        make_float4(silu(g.x) * u.x, silu(g.y) * u.y, silu(g.z) * u.z, silu(g.w) * u.w);
+  } else if (i < n4 + (n & 3u)) {
+    const std::size_t k = 4u * n4 + (i - n4);
+    out[k] = silu(gate[k]) * up[k];
+  }
+}
+
 // Workgroup (four blocks of the row, token t): a wave expands one block, four
 // values a lane (dequant.cuh), and stores 16 bytes a lane at any 4-byte
 // alignment of out. The time is two dependent reads (token, block); against
@@ -271,8 +288,14 @@ extern "C" hipError_t rtxllm_rope_theta(float* vec, uint32_t n_heads, uint32_t h
 extern "C" hipError_t rtxllm_silu_mul(const float* gate, const float* up, size_t n, float* out, hipStream_t stream) {
   if (gate == nullptr || up == nullptr || out == nullptr || n == 0u || n > (std::size_t{1} << 40))
     return hipErrorInvalidValue;
-  hipLaunchKernelGGL(silu_mul_kernel, dim3(static_cast<unsigned>((n + kOpThreads - 1u) / kOpThreads)),
-                     dim3(kOpThreads), 0, stream, gate, up, n, out);
+  const bool vec = ((reinterpret_cast<std::uintptr_t>(gate) | reinterpret_cast<std::uintptr_t>(up) |
+                     reinterpret_cast<std::uintptr_t>(out)) % 16u) == 0u;
+  const std::size_t items = vec ? n / 4u + (n & 3u) : n;
+  const dim3 grid(static_cast<unsigned>((items + kOpThreads - 1u) / kOpThreads));
+  if (vec)
+    hipLaunchKernelGGL(silu_mul_vec_kernel, grid, dim3(kOpThreads), 0, stream, gate, up, n, out);
+  else
+    hipLaunchKernelGGL(silu_mul_kernel, grid, dim3(kOpThreads), 0, stream, gate, up, n, out);
   return hipGetLastError();
 }
 

@@ -81,3 +81,77 @@ def test_dequant_edges_bit_exact(orc, fmt, rows, cols):
         got = big.cpu().numpy()
         assert np.array_equal(got[off:off + n].view(np.uint32), ref.view(np.uint32)), off
         assert np.all(got[:off] == 7.0) and np.all(got[off + n:] == 7.0)
+
+
+@pytest.mark.parametrize("n,count", [(1, 2), (6, 3), (256, 3), (1024, 1), (1028, 130), (4096, 127), (4096, 128),
+                                     (4100, 2), (16384, 2), (16388, 2)])
+@pytest.mark.parametrize("offset", [0, 2])
+def test_rmsnorm_edges(n, count, offset):
+    """Each variant (vector lengths, few and many vectors) and the unaligned
+    fallback, with and without weights, in place, against float64: the fp32 sum
+    of squares (tree) and three roundings give at most 2e-6 relative."""
+    x = packs.normal_f32(n, n * count).reshape(count, n) * np.float32(2.0)
+    w = packs.normal_f32(n + 1, n, mean=1.0, std=0.1)
+    x64 = x.astype(np.float64)
+    norm = x64 / np.sqrt((x64 * x64).mean(1, keepdims=True) + 1e-6)
+    wd = at_offset(w, offset)
+    for weight, ref in ((wd, norm * w), (None, norm)):
+        xd = at_offset(x, offset)
+        out = at_offset(np.zeros_like(x), offset)
+        for dst in (out, xd):  # xd last: in place
+            assert lib().rtxllm_rmsnorm_w(P(xd), P(weight), n, count, 1e-6, P(dst), ops.stream()) == 0
+            np.testing.assert_allclose(dst.cpu().numpy().reshape(count, n), ref, rtol=2e-6)
+
+
+@pytest.mark.parametrize("heads,head_dim,count", [(1, 2, 1), (3, 6, 2), (5, 128, 63), (9, 128, 64), (2, 96, 70),
+                                                  (33, 64, 65), (1, 2048, 64), (1, 2050, 2), (2, 2050, 65)])
+def test_rope_edges(heads, head_dim, count):
+    """One and four pairs a thread, remainders of both, the widest shared-angle
+    head and the one past it, against float64 rotation of the fp32 angle."""
+    theta = 10000.0
+    vec = packs.normal_f32(head_dim, count * heads * head_dim).reshape(count, heads, head_dim // 2, 2)
+    pos = (np.arange(count, dtype=np.uint32) * 37 + 5).astype(np.uint32)
+    freq = np.power(theta, -2.0 * np.arange(head_dim // 2) / head_dim).astype(np.float32)
+    angle = (pos.astype(np.float32)[:, None] * freq).astype(np.float64)[:, None]
+    c, s = np.cos(angle), np.sin(angle)
+    e, o = vec[..., 0].astype(np.float64), vec[..., 1].astype(np.float64)
+    ref = np.stack([e * c - o * s, e * s + o * c], -1)
+    vd, pd = ops.to_dev(vec), ops.to_dev(pos)
+    assert lib().rtxllm_rope_theta(P(vd), heads, head_dim, theta, P(pd), count, ops.stream()) == 0
+    # rounded cos, sin and two products: a few 2^-24 of |(e, o)|; a freq that
+    # rounds the other way moves the angle by its last bit (2^-23 of the angle)
+    tol = 4e-7 * np.abs(vec).max() + 1.3e-7 * float(angle.max()) * np.abs(vec).max() * 0.01
+    np.testing.assert_allclose(vd.cpu().numpy(), ref, rtol=0, atol=tol)
+
+
+@pytest.mark.parametrize("cols", [256, 768, 1024, 1280])
+def test_embed_gather_edges(orc, cols):
+    """Row widths around the four blocks a workgroup holds, unaligned output."""
+    vocab = 50
+    table = packs.synth_raw(F.Q5K, vocab, cols, seed=77)
+    tokens = np.array([49, 0, 50, 7], np.uint32)
+    td, kd = ops.to_dev(table), ops.to_dev(tokens)
+    big = torch.full((len(tokens) * cols + 8,), 7.0, dtype=torch.float32, device="cuda:0")
+    assert lib().rtxllm_embed_gather_q5k(P(td), vocab, cols, P(kd), len(tokens), big.data_ptr() + 4, ops.stream()) == 0
+    got = big.cpu().numpy()
+    assert got[0] == 7.0 and np.all(got[1 + len(tokens) * cols:] == 7.0)
+    got = got[1:1 + len(tokens) * cols].reshape(len(tokens), cols)
+    for i, t in enumerate(tokens):
+        ref = np.empty(cols, np.float32)
+        if t >= vocab:
+            assert np.all(np.isnan(got[i]))
+            continue
+        orc.lib().orc_embed_q5k(orc.ptr(table), cols, int(t), orc.ptr(ref))
+        assert np.array_equal(got[i].view(np.uint32), ref.view(np.uint32)), t
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 1023, 1024, 1027, 4099])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_silu_mul_edges(orc, n, offset):
+    """The vector kernel's remainders, the unaligned fallback, and in place."""
+    g, u = packs.normal_f32(n, n) * np.float32(4.0), packs.normal_f32(n + 1, n)
+    ref = np.empty(n, np.float32)
+    orc.lib().orc_silu_mul(orc.ptr(g), orc.ptr(u), n, orc.ptr(ref))
+    gd, ud = at_offset(g, offset), at_offset(u, 0)
+    assert lib().rtxllm_silu_mul(P(gd), P(ud), n, P(gd), ops.stream()) == 0
+    np.testing.assert_allclose(gd.cpu().numpy(), ref, rtol=2e-6, atol=1e-30)
