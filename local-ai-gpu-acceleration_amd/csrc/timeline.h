@@ -25,7 +25,7 @@
 //   kTlSelfStaged   workgroup * waves_max + wave: a self-staging matvec wave
 //                   has staged its activation groups (the kernel's own region
 //                   holds its entry and end);
-//   kTlRmsStage*    ((seq * blocks + block) * 4 + wave) * 2 + p: entry, end,
+//   kTlRmsStage*    (seq * blocks + block) * 8 + p (one wave): entry, end,
 //                   after the o projection (groups = 1) and after the down
 //                   projection or the embedding (others).
 // Regions 0-15 live in layer.hip's copy of the array, 16-31 in batch.hip's:
