@@ -172,6 +172,7 @@ __global__ __launch_bounds__(kStageThreads) void rms_stage_batch_kernel(RmsStage
 // k (pairs of adjacent rows), q -> q[s], k and v -> the fp16 cache slot of
 // (sequence s, its position); the rule of the batch-1 qkv epilogue.
 struct MmQkv {
+  static constexpr bool kOneTile = true;
   static constexpr int tl_region(int) { return kTlMmQkv; }
   std::uint32_t q_rows, kv_rows, batch, table_stride, rope_positions, group;
   const float2* rope;
@@ -203,6 +204,7 @@ struct MmQkv {
 
 // Interleaved gate / up rows: act[s][i] = silu(gate_i) * up_i.
 struct MmGateUp {
+  static constexpr bool kOneTile = false;
   static constexpr int tl_region(int) { return kTlMmGateUp; }
   float* act;
   std::uint32_t stride;
@@ -218,6 +220,7 @@ struct MmGateUp {
 // A thread keeps the best key of its rows; lanes 8 s .. 8 s + 3 of a wave are
 // sequence s's.
 struct MmLogits {
+  static constexpr bool kOneTile = false;
   static constexpr int tl_region(int) { return kTlMmLogits; }
   float* logits;
   std::uint32_t stride, batch;
@@ -305,6 +308,13 @@ hipError_t launch_mm_epi(const QTensor& w, const void* x16, std::uint32_t batch,
   if (blocks * FmtBytes<FMT>::payload > 0xFFFFFFFFull || blocks * FmtBytes<FMT>::meta > 0xFFFFFFFFull)
     return hipErrorInvalidValue;
   if (geom != nullptr) *geom = g;
+  if constexpr (Epi::kOneTile) {
+    if (g.grid == (w.rows + 15u) / 16u) {  // every tile resident at once
+      hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF, true>), dim3(g.grid, g.groups), dim3(64u * g.ppg), 0, stream, w,
+                         x16, batch, epi);
+      return hipGetLastError();
+    }
+  }
   hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF>), dim3(g.grid, g.groups), dim3(64u * g.ppg), 0, stream, w, x16, batch,
                      epi);
   return hipGetLastError();

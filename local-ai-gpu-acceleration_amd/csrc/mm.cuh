@@ -304,6 +304,7 @@ constexpr int mm_ring() {
 // Plain output: out[pg][s][row] (pg = panel group = blockIdx.y, row stride
 // `stride`): y itself with one panel group, else the groups' partial sums.
 struct MmStore {
+  static constexpr bool kOneTile = true;  // also built for a single tile a workgroup
   static constexpr int tl_region(int fmt) { return fmt_is_iq(fmt) ? kTlMmO : kTlMmDown; }
   float* out;
   std::uint32_t stride, batch;
@@ -323,7 +324,14 @@ struct MmStore {
 // SELF: x16 is instead the fp32 activation [batch][cols], staged by each wave
 // for its own panel with the plain staging rule (block exponent from the
 // block's max |x|, hi / lo fp16 halves), so no staging launch precedes it.
-template <int FMT, class Epi, bool SELF = false>
+// ONE: every workgroup has a single tile (grid = tiles), so its PB units are
+// requested at once and none past them. The ring form requests three units
+// past the last, clamped to it, and each re-read costs the address path as much
+// as a unit: the o projection of the 8B batch-8 step (256 tiles, one a CU) 8.8 ->
+// 7.8 us. With more tiles the re-reads stay: a tail without them for every
+// remainder, run once a launch, cost more in code than it saved (gate_up 21.9
+// -> 22.6 us).
+template <int FMT, class Epi, bool SELF = false, bool ONE = false>
 __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const void* __restrict__ x16,
                                                              std::uint32_t batch, Epi epi) {
   // per-panel partial C of a tile, double buffered by tile parity
@@ -458,9 +466,10 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
     return;
   }
   constexpr int NB = mm_ring<FMT>();
+  static_assert(NB >= PB, "a whole tile in the ring");
   MmRaw ring[NB];
 #pragma unroll
-  for (int j = 0; j < NB - 1; ++j) load_unit(static_cast<std::uint32_t>(j), ring[j]);
+  for (int j = 0; j < (ONE ? PB : NB - 1); ++j) load_unit(static_cast<std::uint32_t>(j), ring[j]);
   if constexpr (!SELF) {
     __builtin_amdgcn_sched_barrier(0);  // the ring's loads ahead of the later blocks' operands
     const uint4* xb = reinterpret_cast<const uint4*>(x16) + PB * panel * 8u * 64u + lane;
@@ -520,7 +529,18 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
     __syncthreads();
     for (std::uint32_t e = threadIdx.x; e < 256u; e += 64u * nw) {  // whole waves
       float v = 0.0f;
-      for (std::uint32_t k = 0; k < nw; ++k) v += red[round & 1u][k][e];
+      if constexpr (fmt_is_iq(FMT)) {
+        for (std::uint32_t k = 0; k < nw; ++k) v += red[round & 1u][k][e];
+      } else {
+        // every panel's read in flight, added in the same order (the LM head of
+        // the 8B batch-8 step 96.5 -> 94.6 us; in the IQ kernels, whose LDS serves
+        // the codebook lookups, it cost gate_up 4 %)
+        float r[kMaxPanels];
+#pragma unroll
+        for (std::uint32_t k = 0; k < kMaxPanels; ++k) r[k] = red[round & 1u][k < nw ? k : nw - 1u][e];
+#pragma unroll
+        for (std::uint32_t k = 0; k < kMaxPanels; ++k) v = k < nw ? v + r[k] : v;
+      }
       const float tot = v + __shfl_xor(v, 4, 64);  // column n ^ 1 is lane l ^ 1 = element e ^ 4
       const float y = tot * t_post;
       const float partner = __shfl_xor(y, 1, 64);  // row ^ 1 is element e ^ 1
@@ -537,17 +557,23 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
   constexpr int PERIOD = NB % PB == 0 ? NB : PB * NB;
   auto step = [&](std::uint32_t u, auto jc) {
     constexpr int j = decltype(jc)::value;
-    load_unit(u + NB - 1u, ring[(j + NB - 1) % NB]);
-    __builtin_amdgcn_sched_barrier(0);  // the prefetch is issued before this unit's work
+    if constexpr (!ONE) {
+      load_unit(u + NB - 1u, ring[(j + NB - 1) % NB]);
+      __builtin_amdgcn_sched_barrier(0);  // the prefetch is issued before this unit's work
+    }
     finish_unit(u, ring[j % NB]);
     if constexpr (j % PB == PB - 1) tile_end(u / PB);
   };
-  std::uint32_t u0 = 0;
-  for (; u0 + PERIOD <= units; u0 += PERIOD)
-    static_for<PERIOD>([&](auto jc) { step(u0 + decltype(jc)::value, jc); });
-  static_for<PERIOD>([&](auto jc) {
-    if (u0 + decltype(jc)::value < units) step(u0 + decltype(jc)::value, jc);
-  });
+  if constexpr (ONE) {
+    static_for<PB>([&](auto jc) { step(decltype(jc)::value, jc); });
+  } else {
+    std::uint32_t u0 = 0;
+    for (; u0 + PERIOD <= units; u0 += PERIOD)
+      static_for<PERIOD>([&](auto jc) { step(u0 + decltype(jc)::value, jc); });
+    static_for<PERIOD>([&](auto jc) {
+      if (u0 + decltype(jc)::value < units) step(u0 + decltype(jc)::value, jc);
+    });
+  }
   epi.finish(wave, lane, nw);
   tl_stamp(kTlR, tl_slot + 15u);
 }

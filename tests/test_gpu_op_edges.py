@@ -155,3 +155,19 @@ def test_silu_mul_edges(orc, n, offset):
     gd, ud = at_offset(g, offset), at_offset(u, 0)
     assert lib().rtxllm_silu_mul(P(gd), P(ud), n, P(gd), ops.stream()) == 0
     np.testing.assert_allclose(gd.cpu().numpy(), ref, rtol=2e-6, atol=1e-30)
+
+
+@pytest.mark.parametrize("fmt", [F.Q4K_RAW, F.Q4K_SPLIT_NATIVE, F.Q5K, F.IQ2S, F.IQ3S], ids=lambda f: F.NAMES[f])
+@pytest.mark.parametrize("cols", [512, 4096])
+def test_batch_single_tile_equals_many_tiles(fmt, cols):
+    """The single-tile kernel (few rows, every tile resident) and the ring over
+    many tiles give a row the same bits; rows % 16 != 0 in both."""
+    rows, few, batch = 70001 if cols == 512 else 16393, 71, 5
+    pack = packs.make_pack(fmt, rows, cols, seed=40 + fmt)
+    blocks = few * (cols // 256)
+    head = packs.Pack(fmt, few, cols, pack.payload[:blocks * F.PAYLOAD_BYTES[fmt]],
+                      None if pack.meta is None else pack.meta[:blocks * F.META_BYTES[fmt]])
+    x16 = ops.stage_batch(ops.to_dev(packs.normal_f32(9, batch * cols).reshape(batch, cols)))
+    many = ops.matvec_batch(ops.DevicePack(pack), x16, batch).cpu().numpy()
+    one = ops.matvec_batch(ops.DevicePack(head), x16, batch).cpu().numpy()
+    assert np.array_equal(many[:, :few].view(np.uint32), one.view(np.uint32))
