@@ -323,8 +323,14 @@ constexpr std::uint32_t kMaxGroup = 8;
 // EARLY_V (the batch launches): the V loads are issued before the scores,
 // which then wait for K and q only; measured faster for eight sequences and
 // slower for one.
-template <int GROUP, bool EARLY_V>
-__global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const _Float16* __restrict__ q, KvLayer kv,
+//
+// QF32 (the standalone entry point): q is the fp32 query [n_kv * GROUP][128] of
+// the sequence, read first and turned into the operand through LDS by the
+// workgroup while K and V are in flight (the q16 rule, so the same scores), in
+// place of a staging launch and its buffer: eight sequences of up to 4096
+// positions 23.0 -> 21.9 us.
+template <int GROUP, bool EARLY_V, bool QF32 = false>
+__global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const void* __restrict__ q_in, KvLayer kv,
                                                                        const std::uint32_t* __restrict__ pos_ptr,
                                                                        std::uint32_t nchunks,
                                                                        float* __restrict__ partials,
@@ -340,7 +346,6 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const _Fl
       (((blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x) * kAttnWaves + (threadIdx.x >> 6)) * 4u;
   tl_stamp(tl_r, tl_slot);
   const std::uint32_t seq = blockIdx.z;
-  q += static_cast<std::size_t>(seq) * q_stride;
   partials += static_cast<std::size_t>(seq) * part_stride;
   const std::int32_t* const table = kv.block_table + static_cast<std::size_t>(seq) * table_stride;
   const std::uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -351,7 +356,15 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const _Fl
   // head n / 2 (hi n even, lo n odd), rows = dims 32 qq + 8 j + i (A's order).
   // Read first: they depend on nothing below.
   uint4 qb[4];
-  {
+  constexpr std::uint32_t kQThreads = GROUP * kHeadDim / 4u;  // QF32: four dims a thread
+  __shared__ __align__(16) _Float16 q16s[QF32 ? kQ16PerKv : 8u];
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  f32x4_any qf;
+  if constexpr (QF32) {
+    const float* qr = static_cast<const float*>(q_in) + static_cast<std::size_t>(seq) * q_stride + g * (GROUP * kHeadDim);
+    qf = *reinterpret_cast<const f32x4_any*>(qr + 4u * (threadIdx.x % kQThreads));  // past them: read again, not used
+  } else {
+    const _Float16* q = static_cast<const _Float16*>(q_in) + static_cast<std::size_t>(seq) * q_stride;
     const uint4* qr = reinterpret_cast<const uint4*>(q + static_cast<std::size_t>(g) * kQ16PerKv) + lane;
 #pragma unroll
     for (int j = 0; j < 4; ++j) qb[j] = qr[64 * j];
@@ -393,6 +406,28 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const _Fl
     vw[j] = *reinterpret_cast<const std::uint32_t*>(kv.v + off + 2u * lane);
   }
   if constexpr (EARLY_V) __builtin_amdgcn_sched_barrier(0);  // every V load issued before the scores
+  if constexpr (QF32) {
+    if (threadIdx.x < kQThreads) {
+      const std::uint32_t h = threadIdx.x / (kHeadDim / 4u), d = 4u * (threadIdx.x % (kHeadDim / 4u));
+#pragma unroll
+      for (std::uint32_t i = 0; i < 4u; ++i) {
+        float x = qf[i] * 0.08838834764831845f;  // 1 / sqrt(128)
+        // one rounded x for hi and lo: left to itself the compiler rounds the
+        // product to fp16 once for lo's hi and by way of fp32 for the stored one
+        asm("" : "+v"(x));
+        const _Float16 hi = static_cast<_Float16>(x);
+        const std::size_t k = q16_index(0u, h, d + i, 0u);
+        q16s[k] = hi;
+        q16s[k + 8u] = static_cast<_Float16>(x - static_cast<float>(hi));
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint4 t = reinterpret_cast<const uint4*>(q16s)[64 * j + lane];
+      qb[j] = r < 2u * GROUP ? t : make_uint4(0u, 0u, 0u, 0u);  // columns without a head
+    }
+  }
   f32x4 sc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
   for (int j = 0; j < 4; ++j)
@@ -718,7 +753,7 @@ std::size_t attention_partials_floats(std::uint32_t n_heads, std::uint32_t n_kv,
   return static_cast<std::size_t>(n_kv) * nchunks * (n_heads / n_kv) * (kHeadDim + 2u);
 }
 
-hipError_t launch_attention_batch(const void* q, const KvLayer& kv, std::uint32_t n_heads, const std::uint32_t* pos,
+hipError_t launch_attention_batch(const void* q, bool q_f32, const KvLayer& kv, std::uint32_t n_heads, const std::uint32_t* pos,
                                   std::uint32_t span, std::uint32_t batch, std::uint32_t table_stride,
                                   float* partials, float* att, void* xq_att, void* x16_att, hipStream_t stream) {
   if (kv.n_kv == 0u || n_heads % kv.n_kv != 0u || n_heads / kv.n_kv > kMaxGroup || kv.capacity == 0u ||
@@ -733,16 +768,22 @@ hipError_t launch_attention_batch(const void* q, const KvLayer& kv, std::uint32_
   const std::uint32_t nchunks = (span + kAttnChunk - 1u) / kAttnChunk;
   const std::size_t part = attention_partials_floats(n_heads, kv.n_kv, span);
   if (part > 0xFFFFFFFFull) return hipErrorInvalidValue;
-  const std::uint32_t part_stride = static_cast<std::uint32_t>(part), q_stride = kv.n_kv * kQ16PerKv;
+  const std::uint32_t part_stride = static_cast<std::uint32_t>(part);
+  const std::uint32_t q_stride = q_f32 ? n_heads * kHeadDim : kv.n_kv * kQ16PerKv;
   const dim3 grid(nchunks, kv.n_kv, batch), block(64 * kAttnWaves);
-#define RTXLLM_ATTN_CASE(G)                                                                                      \
-  case G:                                                                                                        \
-    if (batch > 1u)                                                                                              \
-      hipLaunchKernelGGL((attn_partial_kernel<G, true>), grid, block, 0, stream, static_cast<const _Float16*>(q), \
-                         kv, pos, nchunks, partials, q_stride, table_stride, part_stride);                      \
-    else                                                                                                         \
-      hipLaunchKernelGGL((attn_partial_kernel<G, false>), grid, block, 0, stream, static_cast<const _Float16*>(q), \
-                         kv, pos, nchunks, partials, q_stride, table_stride, part_stride);                      \
+#define RTXLLM_ATTN_LAUNCH(G, EARLY_V, QF32)                                                                       \
+  hipLaunchKernelGGL((attn_partial_kernel<G, EARLY_V, QF32>), grid, block, 0, stream, q, kv, pos, nchunks, partials, \
+                     q_stride, table_stride, part_stride)
+#define RTXLLM_ATTN_CASE(G)                            \
+  case G:                                              \
+    if (q_f32 && batch > 1u)                           \
+      RTXLLM_ATTN_LAUNCH(G, true, true);               \
+    else if (q_f32)                                    \
+      RTXLLM_ATTN_LAUNCH(G, false, true);              \
+    else if (batch > 1u)                               \
+      RTXLLM_ATTN_LAUNCH(G, true, false);              \
+    else                                               \
+      RTXLLM_ATTN_LAUNCH(G, false, false);             \
     break;
   switch (group) {
     RTXLLM_ATTN_CASE(1)
@@ -752,6 +793,7 @@ hipError_t launch_attention_batch(const void* q, const KvLayer& kv, std::uint32_
     default: return hipErrorInvalidValue;
   }
 #undef RTXLLM_ATTN_CASE
+#undef RTXLLM_ATTN_LAUNCH
   hipError_t st = hipGetLastError();
   if (st != hipSuccess) return st;
   if (x16_att != nullptr) {
@@ -768,7 +810,7 @@ hipError_t launch_attention_batch(const void* q, const KvLayer& kv, std::uint32_
 hipError_t launch_attention(const void* q, const KvLayer& kv, std::uint32_t n_heads, const std::uint32_t* pos,
                             std::uint32_t span, float* partials, float* att, void* xq_att, hipStream_t stream) {
   if (xq_att == nullptr) return hipErrorInvalidValue;
-  return launch_attention_batch(q, kv, n_heads, pos, span, 1u, 0u, partials, att, xq_att, nullptr, stream);
+  return launch_attention_batch(q, false, kv, n_heads, pos, span, 1u, 0u, partials, att, xq_att, nullptr, stream);
 }
 
 hipError_t launch_residual(int fmt, const std::uint8_t* payload, const std::uint8_t* meta, std::uint32_t rows,

@@ -195,28 +195,6 @@ __global__ __launch_bounds__(256) void embed_gather_q5k_kernel(const std::uint8_
   *reinterpret_cast<f32x4_any*>(out + static_cast<std::size_t>(t) * cols + 256u * b + 4u * lane) = v;
 }
 
-// fp32 queries q [count][n_heads][128] -> the attention's query operand (q16):
-// one thread per fp16 slot of the operand image of one vector (n_kv * 2048
-// slots; slot = ((g * 4 + j) * 64 + l) * 8 + i holds dim 32 (l / 16) + 8 j + i
-// of column n = l % 16 = 2 h + part of kv head g, zero for h >= group).
-__global__ __launch_bounds__(kOpThreads) void q16_stage_kernel(const float* __restrict__ q, std::uint32_t n_kv,
-                                                               std::uint32_t group, _Float16* __restrict__ q16) {
-  const std::uint32_t slots = n_kv * (kQ16PerKv);
-  const std::uint32_t idx = blockIdx.x * kOpThreads + threadIdx.x;
-  if (idx >= slots) return;
-  const std::uint32_t r = blockIdx.y;
-  const std::uint32_t i = idx & 7u, l = (idx >> 3) & 63u, j = (idx >> 9) & 3u, g = idx >> 11;
-  const std::uint32_t d = 32u * (l >> 4) + 8u * j + i, n = l & 15u, h = n >> 1, part = n & 1u;
-  _Float16 v = static_cast<_Float16>(0.0f);
-  if (h < group) {
-    const float x = q[(static_cast<std::size_t>(r) * n_kv * group + g * group + h) * kHeadDim + d] *
-                    0.08838834764831845f;  // 1 / sqrt(128)
-    const _Float16 hi = static_cast<_Float16>(x);
-    v = part == 0u ? hi : static_cast<_Float16>(x - static_cast<float>(hi));
-  }
-  q16[static_cast<std::size_t>(r) * slots + idx] = v;
-}
-
 // One workgroup per vector (argmax.cuh).
 template <std::uint32_t U>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(const float* __restrict__ x, std::uint32_t n,
@@ -313,6 +291,8 @@ extern "C" hipError_t rtxllm_embed_gather_q5k(const uint8_t* table, uint32_t voc
 extern "C" size_t rtxllm_attn_decode_workspace(uint32_t n_heads, uint32_t n_kv_heads, uint32_t capacity,
                                                uint32_t count) {
   if (!group_ok(n_heads, n_kv_heads) || capacity == 0u || count == 0u) return 0u;
+  // the partials; the first term is room that an earlier staging of q needed and
+  // that callers' buffers have
   return align256(static_cast<std::size_t>(count) * n_kv_heads * kQ16BytesPerKv) +
          4u * static_cast<std::size_t>(count) * attention_partials_floats(n_heads, n_kv_heads, capacity);
 }
@@ -331,14 +311,7 @@ extern "C" hipError_t rtxllm_attn_decode_gqa_f16(const float* q, const uint16_t*
     return hipErrorInvalidValue;
   const std::size_t need = rtxllm_attn_decode_workspace(n_heads, n_kv_heads, capacity, count);
   if (need == 0u || workspace_bytes < need) return hipErrorInvalidValue;
-  auto* q16 = static_cast<_Float16*>(workspace);
-  auto* partials = reinterpret_cast<float*>(static_cast<std::uint8_t*>(workspace) +
-                                            align256(static_cast<std::size_t>(count) * n_kv_heads * kQ16BytesPerKv));
-  const std::uint32_t slots = n_kv_heads * kQ16PerKv;
-  hipLaunchKernelGGL(q16_stage_kernel, dim3((slots + kOpThreads - 1u) / kOpThreads, count), dim3(kOpThreads), 0, stream,
-                     q, n_kv_heads, n_heads / n_kv_heads, q16);
-  hipError_t st = hipGetLastError();
-  if (st != hipSuccess) return st;
+  auto* partials = static_cast<float*>(workspace);
   KvLayer kv{};
   kv.k = const_cast<std::uint16_t*>(k_cache);
   kv.v = const_cast<std::uint16_t*>(v_cache);
@@ -346,7 +319,7 @@ extern "C" hipError_t rtxllm_attn_decode_gqa_f16(const float* q, const uint16_t*
   kv.page_size = page_size;
   kv.n_kv = n_kv_heads;
   kv.capacity = capacity;
-  return launch_attention_batch(q16, kv, n_heads, pos, capacity, count, table_stride, partials, out, nullptr, nullptr,
+  return launch_attention_batch(q, true, kv, n_heads, pos, capacity, count, table_stride, partials, out, nullptr, nullptr,
                                 stream);
 }
 

@@ -171,3 +171,41 @@ def test_batch_single_tile_equals_many_tiles(fmt, cols):
     many = ops.matvec_batch(ops.DevicePack(pack), x16, batch).cpu().numpy()
     one = ops.matvec_batch(ops.DevicePack(head), x16, batch).cpu().numpy()
     assert np.array_equal(many[:, :few].view(np.uint32), one.view(np.uint32))
+
+
+@pytest.mark.parametrize("heads,n_kv", [(1, 1), (6, 3), (4, 1), (16, 2)])
+@pytest.mark.parametrize("count", [1, 3])
+def test_attention_fp32_queries_unaligned(orc, heads, n_kv, count):
+    """Each group size with the workgroup's own staging of q (few kv heads, a short
+    last chunk, a single position), q off its 16-byte alignment, and a capacity
+    that is no multiple of the 128-position chunk."""
+    hd, page, cap = 128, 16, 304
+    pps = cap // page
+    npages = count * pps
+    positions = np.array([303, 0, 129][:count], np.uint32)
+    table = np.array([(5 * i + 3) % npages for i in range(npages)], np.int32)
+    assert len(set(table.tolist())) == npages
+    k = packs.normal_f16_bits(81, npages * n_kv * page * hd)
+    v = packs.normal_f16_bits(82, npages * n_kv * page * hd)
+    q = packs.normal_f32(83, count * heads * hd)
+    qd, kd, vd = at_offset(q, 1), ops.to_dev(k), ops.to_dev(v)
+    td, pd = ops.to_dev(table), ops.to_dev(positions)
+    need = int(lib().rtxllm_attn_decode_workspace(heads, n_kv, cap, count))
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda:0")
+    out = torch.empty(count * heads * hd, dtype=torch.float32, device="cuda:0")
+    assert lib().rtxllm_attn_decode_gqa_f16(P(qd), P(kd), P(vd), P(td), pps, heads, n_kv, page, cap, P(pd), count,
+                                            P(out), P(ws), need, ops.stream()) == 0
+    got = out.cpu().numpy().reshape(count, heads, hd).astype(np.float64)
+    kf = k.view(np.float16).reshape(npages, n_kv, page, hd).astype(np.float64)
+    vf = v.view(np.float16).reshape(npages, n_kv, page, hd).astype(np.float64)
+    for r in range(count):
+        rows = table[r * pps:(r + 1) * pps]
+        n = int(positions[r]) + 1
+        for h in range(heads):
+            g = h // (heads // n_kv)
+            ks, vs = (t[rows, g].reshape(cap, hd)[:n] for t in (kf, vf))
+            s = ks @ (q.reshape(count, heads, hd)[r, h].astype(np.float64) / np.sqrt(128.0))
+            p = np.exp(s - s.max())
+            ref = (p / p.sum()) @ vs
+            # q enters as an fp16 hi / lo pair (~22 bits); scores up to ~40
+            np.testing.assert_allclose(got[r, h], ref, rtol=0, atol=1e-5 * np.abs(ref).max())
