@@ -209,3 +209,19 @@ def test_attention_fp32_queries_unaligned(orc, heads, n_kv, count):
             ref = (p / p.sum()) @ vs
             # q enters as an fp16 hi / lo pair (~22 bits); scores up to ~40
             np.testing.assert_allclose(got[r, h], ref, rtol=0, atol=1e-5 * np.abs(ref).max())
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 3), (3, 5), (4, 1024), (7, 1025), (4096, 100), (4099, 4097),
+                                       (16384, 1000), (16387, 17000)])
+@pytest.mark.parametrize("offset", [0, 3])
+def test_rmsnorm_feedback_edges(rows, cols, offset):
+    """Remainders of the vector loads and of their steps, unaligned logits, fewer
+    and more columns than rows, against float64: the fp32 sum (tree), rsqrtf and
+    two roundings give at most 2e-6 relative."""
+    x = packs.normal_f32(rows, rows) * np.float32(3.0)
+    x64 = x.astype(np.float64)
+    ref = (x64 / np.sqrt((x64 * x64).mean() + 1e-6))[np.arange(cols) % rows]
+    act = torch.empty(cols, dtype=torch.float32, device="cuda:0")
+    xd = at_offset(x, offset)
+    assert lib().rtxllm_launch_rmsnorm_feedback(P(xd), P(act), rows, cols, 1e-6, ops.stream()) == 0
+    np.testing.assert_allclose(act.cpu().numpy(), ref, rtol=2e-6)
