@@ -720,6 +720,7 @@ struct EpiWaves<E, std::void_t<decltype(E::kWaves)>> {
 // the prologue, instead of every wave loading its own slice: the CU's load
 // path then carries the activation once per workgroup.
 constexpr std::uint32_t kShareXCols = 4096;
+constexpr std::uint32_t kSelfShareCols = 8192;
 template <class E, class = void>
 struct EpiShareX {
   static constexpr bool value = false;
@@ -790,7 +791,13 @@ __device__ __forceinline__ void pair_publish(std::uint32_t* counter, std::uint32
 //    GR / TILE). Results collect in LDS, and after the group's last round wave 0
 //    hands all GR of them to epi.group(), inside the workgroup: no other
 //    workgroup's results are needed, so no device-wide synchronisation.
-template <int FMT, int UPL, int TILE, bool SELF, class Epi>
+// SHARE (self-staging, plain epilogues, at most kSelfShareCols columns): the
+// workgroup stages x once, four values a thread, into LDS, and every row group
+// reads its digits there. Otherwise each wave converts its own columns, 2 x 16
+// values a lane (~350 VALU), which for a launch of one or two tiles a wave is
+// as much work as a tile: IQ2_S 14336 x 4096 from fp32 x 14.1 -> 9.8 us (the
+// rule and its figures: mv_share_groups).
+template <int FMT, int UPL, int TILE, bool SELF, class Epi, bool SHARE = false>
 __global__ __launch_bounds__(64 * EpiWaves<Epi>::value) void mv_kernel(QTensor w, XSrc xs, std::uint32_t rows,
                                                                       std::uint32_t ks, Epi epi_arg) {
   static_assert(Epi::kTile == TILE, "epilogue tile");
@@ -811,8 +818,11 @@ __global__ __launch_bounds__(64 * EpiWaves<Epi>::value) void mv_kernel(QTensor w
   // Pairwise hand-over: ready[w] = rounds wave w has published, taken[w] =
   // rounds the row group's epilogue wave w has consumed.
   __shared__ std::uint32_t ready[kPair ? WMAX : 1u], taken[kPair ? WMAX : 1u];
-  // The workgroup's copy of the staged x (kShareX), in its global layout.
-  constexpr std::uint32_t kXPieces = kShareX ? static_cast<std::uint32_t>(xq_bytes(kShareXCols) / 16u) : 1u;
+  static_assert(!SHARE || (SELF && UPL == 1 && GR == 0u && !kPair), "shared self-staging");
+  // The workgroup's copy of the staged x (kShareX, SHARE), in its global layout.
+  constexpr std::uint32_t kXPieces =
+      kShareX ? static_cast<std::uint32_t>(xq_bytes(kShareXCols) / 16u)
+              : (SHARE ? static_cast<std::uint32_t>(xq_bytes(kSelfShareCols) / 16u) : 1u);
   __shared__ uint4 xshare[kXPieces];
   // Grouped epilogues: a group's results, double buffered by group parity.
   __shared__ float gbuf[2][GR > 0u ? GR : 1u];
@@ -906,11 +916,24 @@ __global__ __launch_bounds__(64 * EpiWaves<Epi>::value) void mv_kernel(QTensor w
   // request wait for these loads.
   XG x0[UPL], x1[UPL];
   f32x16 xf0[UPL], xf1[UPL];
+  // SHARE: quads of four values tid, tid + threads, ...: the first two a thread
+  // here (all of them, up to 8 values a thread), any others below
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  const std::uint32_t quads = w.cols / 4u;
+  f32x4_any xq4[SHARE ? 2 : 1];
+  if constexpr (SHARE) {
+#pragma unroll
+    for (std::uint32_t j = 0; j < 2u; ++j) {
+      const std::uint32_t c = threadIdx.x + j * blockDim.x;
+      xq4[j] = *reinterpret_cast<const f32x4_any*>(xs.x + 4u * (c < quads ? c : quads - 1u));
+    }
+  }
 #pragma unroll
   for (int i = 0; i < UPL; ++i) {
     std::uint32_t g0, g1;
     unit_groups<FMT>(ub[i], uk[i], g0, g1);
-    if constexpr (SELF) {
+    if constexpr (SHARE) {
+    } else if constexpr (SELF) {
       if (xs.x_aligned != 0u) {
         xf0[i] = xg_read<true>(xs.x, g0);
         xf1[i] = xg_read<true>(xs.x, g1);
@@ -927,7 +950,28 @@ __global__ __launch_bounds__(64 * EpiWaves<Epi>::value) void mv_kernel(QTensor w
   // each row group keeps one tile of weights in flight.
   UnitRaw buf[2][TILE][UPL];
   load_tile(tile_of(0u), buf[0]);
-  if constexpr (SELF) {
+  if constexpr (SHARE) {
+    __builtin_amdgcn_sched_barrier(0);  // every load of the first tile issued before the conversion
+    std::uint8_t* const xb = reinterpret_cast<std::uint8_t*>(xshare);
+    const std::uint32_t cols = w.cols;
+    auto put = [&](std::uint32_t c, const f32x4_any& t) {
+      const float v[4] = {t.x, t.y, t.z, t.w};
+      const XQuad g = quant4(v);  // quads is a multiple of 64: whole waves are in or out
+      if (c >= quads) return;
+      *reinterpret_cast<std::uint32_t*>(xb + 4u * c) = g.h;
+      *reinterpret_cast<std::uint32_t*>(xb + cols + 4u * c) = g.m;
+      *reinterpret_cast<std::uint32_t*>(xb + 2u * cols + 4u * c) = g.l;
+      if ((c & 3u) == 0u) {
+        float* const sx = reinterpret_cast<float*>(xb + 3u * cols);
+        sx[c >> 2] = g.s;
+        sx[cols / kXGroup + (c >> 2)] = g.sum;
+      }
+    };
+#pragma unroll
+    for (std::uint32_t j = 0; j < 2u; ++j) put(threadIdx.x + j * blockDim.x, xq4[j]);
+    for (std::uint32_t c = threadIdx.x + 2u * blockDim.x; c < quads; c += blockDim.x)
+      put(c, *reinterpret_cast<const f32x4_any*>(xs.x + 4u * c));
+  } else if constexpr (SELF) {
     __builtin_amdgcn_sched_barrier(0);  // every load of the first tile issued before the conversion
 #pragma unroll
     for (int i = 0; i < UPL; ++i) {
@@ -950,8 +994,8 @@ __global__ __launch_bounds__(64 * EpiWaves<Epi>::value) void mv_kernel(QTensor w
       xshare[c] = reinterpret_cast<const uint4*>(xs.xq.h)[c];
   }
   if constexpr (fmt_is_iq(FMT)) lds_grid_commit(*tables, grid_stage, iq_image<FMT>(), threadIdx.x, blockDim.x);
-  else if constexpr (kPair || kShareX) __syncthreads();
-  if constexpr (kShareX) {
+  else if constexpr (kPair || kShareX || SHARE) __syncthreads();
+  if constexpr (kShareX || SHARE) {
     // the staged layout (h, m, l: cols bytes each; s, sum: cols / 16 floats)
     const std::uint8_t* xb = reinterpret_cast<const std::uint8_t*>(xshare);
     const std::uint32_t c = w.cols;

@@ -42,9 +42,11 @@ struct MvGeom {
 };
 
 // resident(block_threads) = workgroups of that size resident per CU (0: unknown).
+// share > 0: the shared self-staging kernel with that many row groups a workgroup
+// (mv_share_groups), the rest as the plain launches.
 template <class Resident>
 inline bool mv_geom(int fmt, std::uint32_t rows, std::uint32_t cols, int tile, std::uint32_t group_rows,
-                    std::uint32_t max_waves, Resident resident, MvGeom& g) {
+                    std::uint32_t max_waves, std::uint32_t share, Resident resident, MvGeom& g) {
   const std::uint32_t units = cols / 32u;
   g.upl = units > 512u ? 2 : 1;
   g.ks = (units + 64u * g.upl - 1u) / (64u * g.upl);
@@ -60,6 +62,7 @@ inline bool mv_geom(int fmt, std::uint32_t rows, std::uint32_t cols, int tile, s
     grid = (tiles + tg - 1u) / tg;
   } else {
     g.nrg = g.ks >= 4u ? 1u : 4u / g.ks;
+    if (share > 0u) g.nrg = share;
     grid = (tiles + g.nrg - 1) / g.nrg;
   }
   const std::uint32_t per_cu = static_cast<std::uint32_t>(resident(64u * g.ks * g.nrg));
@@ -72,7 +75,7 @@ inline bool mv_geom(int fmt, std::uint32_t rows, std::uint32_t cols, int tile, s
     if (group_rows == 0u && per_cu_wide > 0u) {
       g.nrg = nrg_wide;
       grid = per_cu_wide * cus;
-    } else if (group_rows == 0u && fmt_is_iq(fmt) && g.nrg > 1u) {
+    } else if (group_rows == 0u && share == 0u && fmt_is_iq(fmt) && g.nrg > 1u) {
       g.nrg = 1u;
       const std::uint32_t per_cu1 = static_cast<std::uint32_t>(resident(64u * g.ks));
       grid = (per_cu1 > 0u ? per_cu1 : 1u) * cus;
@@ -86,7 +89,7 @@ inline bool mv_geom(int fmt, std::uint32_t rows, std::uint32_t cols, int tile, s
 
 // Resident workgroups per CU of one mv_kernel instantiation at a block size
 // (cached; 0 if the query fails).
-template <int FMT, int UPL, int TILE, bool SELF, class Epi>
+template <int FMT, int UPL, int TILE, bool SELF, class Epi, bool SHARE = false>
 inline int mv_resident(std::uint32_t block_threads) {
   constexpr std::uint32_t kW = EpiWaves<Epi>::value;
   static int cache[kW + 1] = {};
@@ -95,7 +98,7 @@ inline int mv_resident(std::uint32_t block_threads) {
   if (cache[w] == 0) {
     int n = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(
-            &n, reinterpret_cast<const void*>(&mv_kernel<FMT, UPL, TILE, SELF, Epi>),
+            &n, reinterpret_cast<const void*>(&mv_kernel<FMT, UPL, TILE, SELF, Epi, SHARE>),
             static_cast<int>(block_threads), 0) != hipSuccess || n <= 0)
       return 0;
     cache[w] = n;
@@ -103,14 +106,43 @@ inline int mv_resident(std::uint32_t block_threads) {
   return cache[w];
 }
 
+// Row groups per workgroup of the shared self-staging kernel (0: the kernel whose
+// waves stage their own columns). Same results bit for bit, so the line is drawn
+// by time alone (fp32 x, cold weights, us of each without / with sharing):
+//  * IQ formats, up to 8 waves a workgroup: IQ2_S 8192x2048 7.7 / 5.5, 14336x4096
+//    14.1 / 9.8, 4096x8192 11.8 / 8.6; IQ3_S 7.2 / 6.0, 13.2 / 11.1, 10.2 / 9.3;
+//  * K-quants only where one wave holds a row (Q5_K 8192x2048 5.7 / 5.5), Q4_K up
+//    to 1024 columns (30001x1024 9.6 / 9.1; 8192x2048 5.1 / 5.2); with two waves
+//    a row the barrier costs more (Q4_K 4096x4096 5.2 / 6.0);
+//  * not from four rounds a row group on, where the staging is paid off anyway
+//    and the row groups of a workgroup run in step (IQ3_S 64000x2560 29.3 / 31.3);
+//  * no more row groups than keep a workgroup on every CU (IQ3_S 4096x1024 4.5 /
+//    4.8 with eight on half of the CUs, 4.1 with four), and none where that
+//    leaves several waves one row group to stage for (2000x8192 7.3 / 8.2).
+template <int FMT, bool SELF, class Epi>
+inline std::uint32_t mv_share_groups(std::uint32_t rows, std::uint32_t cols) {
+  if constexpr (!SELF || EpiGroupRows<Epi>::value > 0u) return 0u;
+  const std::uint32_t ks = (cols / 32u + 63u) / 64u, cus = static_cast<std::uint32_t>(num_cus());
+  const std::uint32_t tiles = (rows + Epi::kTile - 1u) / Epi::kTile;
+  const bool k_quant = ks == 1u && (FMT == RTXLLM_FMT_Q5K || cols <= 1024u);
+  const std::uint32_t most = fmt_is_iq(FMT) ? 8u / ks : (k_quant ? 4u : 0u);
+  // 16 waves a CU resident: 16 / ks row groups
+  if (cols > kSelfShareCols || most == 0u || static_cast<std::uint64_t>(tiles) * ks > 4ull * 16ull * cus) return 0u;
+  const std::uint32_t fill = tiles / cus < 1u ? 1u : tiles / cus;
+  const std::uint32_t groups = fill < most ? fill : most;
+  return groups == 1u && ks > 1u ? 0u : groups;
+}
+
 template <int FMT, bool SELF, class Epi>
 inline bool mv_geometry_fmt(std::uint32_t rows, std::uint32_t cols, MvGeom& g) {
   constexpr int kT = Epi::kTile;
-  const std::uint32_t units = cols / 32u;
-  auto resident = [units](std::uint32_t threads) {
+  constexpr bool kCanShare = SELF && EpiGroupRows<Epi>::value == 0u;
+  const std::uint32_t units = cols / 32u, share = mv_share_groups<FMT, SELF, Epi>(rows, cols);
+  auto resident = [units, share](std::uint32_t threads) {
+    if (kCanShare && share > 0u) return mv_resident<FMT, 1, kT, SELF, Epi, kCanShare>(threads);
     return units > 512u ? mv_resident<FMT, 2, kT, SELF, Epi>(threads) : mv_resident<FMT, 1, kT, SELF, Epi>(threads);
   };
-  return mv_geom(FMT, rows, cols, kT, EpiGroupRows<Epi>::value, EpiWaves<Epi>::value, resident, g);
+  return mv_geom(FMT, rows, cols, kT, EpiGroupRows<Epi>::value, EpiWaves<Epi>::value, share, resident, g);
 }
 
 template <int FMT, bool SELF, class Epi>
@@ -124,6 +156,12 @@ inline hipError_t launch_mv_fmt(const QTensor& w, const XSrc& xs, std::uint32_t 
   MvGeom g;
   if (!mv_geometry_fmt<FMT, SELF, Epi>(row_count, w.cols, g)) return hipErrorInvalidValue;
   const dim3 grid(g.grid), block(64u * g.ks * g.nrg);
+  if constexpr (SELF && EpiGroupRows<Epi>::value == 0u) {
+    if (mv_share_groups<FMT, SELF, Epi>(row_count, w.cols) > 0u) {
+      hipLaunchKernelGGL((mv_kernel<FMT, 1, kT, SELF, Epi, true>), grid, block, 0, stream, w, xs, row_count, g.ks, epi);
+      return hipGetLastError();
+    }
+  }
   if (g.upl == 2) {
     hipLaunchKernelGGL((mv_kernel<FMT, 2, kT, SELF, Epi>), grid, block, 0, stream, w, xs, row_count, g.ks, epi);
   } else {

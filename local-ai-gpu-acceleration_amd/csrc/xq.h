@@ -144,6 +144,50 @@ __device__ __forceinline__ void quant16(const float v[16], XG& g) {
   g.sum = g.s * static_cast<float>(total);
 }
 
+// quant16 spread over four adjacent lanes, each with four values of the group
+// (every lane of the wave active): the group's maximum, NaN flag and integer sum
+// by quad exchanges (order-free), so the digits, scale and sum equal quant16's.
+// Lane (lane & 3) gets its values' digit words; s and sum are the group's in all.
+struct XQuad {
+  std::uint32_t h, m, l;
+  float s, sum;
+};
+__device__ __forceinline__ std::uint32_t xq_quad_dpp1(std::uint32_t v) {
+  return static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, false));
+}
+__device__ __forceinline__ std::uint32_t xq_quad_dpp2(std::uint32_t v) {
+  return static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false));
+}
+__device__ __forceinline__ XQuad quant4(const float v[4]) {
+  float m = fmaxf(fmaxf(fmaxf(0.0f, fabsf(v[0])), fmaxf(fabsf(v[1]), fabsf(v[2]))), fabsf(v[3]));
+  std::uint32_t nan = __builtin_isunordered(v[0], v[1]) || __builtin_isunordered(v[2], v[3]) ? 1u : 0u;
+  m = fmaxf(m, __uint_as_float(xq_quad_dpp1(__float_as_uint(m))));
+  m = fmaxf(m, __uint_as_float(xq_quad_dpp2(__float_as_uint(m))));
+  nan |= xq_quad_dpp1(nan);
+  nan |= xq_quad_dpp2(nan);
+  const XScale sc = xq_scale(m, nan != 0u);
+  std::uint32_t Y[4], total = 0u;
+#pragma unroll
+  for (int b = 0; b < 4; ++b) {
+    const int X = xq_fixed(v[b], sc);
+    total += static_cast<std::uint32_t>(X);
+    Y[b] = static_cast<std::uint32_t>(X + kXQBias);
+  }
+  total += xq_quad_dpp1(total);
+  total += xq_quad_dpp2(total);
+  const std::uint32_t p01 = __builtin_amdgcn_perm(Y[1], Y[0], 0x05010400u);  // as in quant16
+  const std::uint32_t p23 = __builtin_amdgcn_perm(Y[3], Y[2], 0x05010400u);
+  const std::uint32_t q01 = __builtin_amdgcn_perm(Y[1], Y[0], 0x06020602u);
+  const std::uint32_t q23 = __builtin_amdgcn_perm(Y[3], Y[2], 0x06020602u);
+  XQuad r;
+  r.l = __builtin_amdgcn_perm(p23, p01, 0x05040100u) ^ 0x80808080u;
+  r.m = __builtin_amdgcn_perm(p23, p01, 0x07060302u) ^ 0x80808080u;
+  r.h = __builtin_amdgcn_perm(q23, q01, 0x05040100u);
+  r.s = sc.s;
+  r.sum = sc.s * static_cast<float>(static_cast<int>(total));
+  return r;
+}
+
 __device__ __forceinline__ void xg_load(const XQ& x, std::uint32_t group, XG& g) {
   const uint4 h = *reinterpret_cast<const uint4*>(x.h + kXGroup * group);
   const uint4 m = *reinterpret_cast<const uint4*>(x.m + kXGroup * group);

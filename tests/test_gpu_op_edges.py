@@ -225,3 +225,28 @@ def test_rmsnorm_feedback_edges(rows, cols, offset):
     xd = at_offset(x, offset)
     assert lib().rtxllm_launch_rmsnorm_feedback(P(xd), P(act), rows, cols, 1e-6, ops.stream()) == 0
     np.testing.assert_allclose(act.cpu().numpy(), ref, rtol=2e-6)
+
+
+@pytest.mark.parametrize("fmt", [F.Q4K_SPLIT_NATIVE, F.Q4K_SPLIT_COMPACT, F.Q5K, F.IQ2S, F.IQ3S, F.IQ2S_UNITS,
+                                 F.IQ3S_UNITS], ids=lambda f: F.NAMES[f])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (1023, 512), (1030, 1024), (2049, 2048), (2055, 2304), (4097, 4096),
+                                       (8195, 4352), (2048, 8192), (2051, 8448), (4099, 8192), (70001, 256)])
+def test_matvec_shared_staging_equals_staged_input(fmt, rows, cols):
+    """One to eight row groups a workgroup share the staging of an fp32 x, or none
+    do (widths, row counts and formats on both sides of the rule): always the
+    bits of rtxllm_stage_activation + rtxllm_matvec_xq, x aligned or not, and a
+    NaN or infinite value poisons as there."""
+    pack = packs.make_pack(fmt, rows, cols, seed=300 + fmt)
+    w = ops.DevicePack(pack)
+    x = packs.normal_f32(cols, cols)
+    x[16:32] = 0.0
+    x[40] *= np.float32(1e4)
+    for bad in (None, np.nan, np.inf):
+        if bad is not None:
+            x[cols - 5] = bad
+        ref = ops.matvec_xq(w, ops.stage(ops.to_dev(x))).cpu().numpy()
+        for off in (0, 1):
+            y = torch.empty(rows, dtype=torch.float32, device="cuda:0")
+            xd = at_offset(x, off)
+            assert lib().rtxllm_matvec(fmt, P(w.payload), P(w.meta), P(xd), P(y), rows, cols, ops.stream()) == 0
+            assert np.array_equal(y.cpu().numpy().view(np.uint32), ref.view(np.uint32)), (bad, off)
