@@ -256,8 +256,11 @@ int mm_resident(std::uint32_t threads) {
   if (w == 0u || w > kMaxPanels) return 0;
   if (cache[w] == 0) {
     int n = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, reinterpret_cast<const void*>(&mm_kernel<FMT, Epi, SELF>),
-                                                     static_cast<int>(threads), 0) != hipSuccess || n <= 0)
+    // the kernel of a persistent grid (a single-tile grid takes its geometry)
+    const void* f = reinterpret_cast<const void*>(&mm_kernel<FMT, Epi, SELF>);
+    if constexpr (mm_lds_fits<FMT, SELF>(kMaxPanels, false))
+      if (mm_lds_fits<FMT, SELF>(w, false)) f = reinterpret_cast<const void*>(&mm_kernel<FMT, Epi, SELF, false, true>);
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, static_cast<int>(threads), 0) != hipSuccess || n <= 0)
       return 0;
     cache[w] = n;
   }
@@ -308,15 +311,22 @@ hipError_t launch_mm_epi(const QTensor& w, const void* x16, std::uint32_t batch,
   if (blocks * FmtBytes<FMT>::payload > 0xFFFFFFFFull || blocks * FmtBytes<FMT>::meta > 0xFFFFFFFFull)
     return hipErrorInvalidValue;
   if (geom != nullptr) *geom = g;
-  if constexpr (Epi::kOneTile) {
-    if (g.grid == (w.rows + 15u) / 16u) {  // every tile resident at once
-      hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF, true>), dim3(g.grid, g.groups), dim3(64u * g.ppg), 0, stream, w,
-                         x16, batch, epi);
+  const dim3 grid(g.grid, g.groups), block(64u * g.ppg);
+  const bool one = Epi::kOneTile && g.grid == (w.rows + 15u) / 16u;  // every tile resident
+  if constexpr (mm_lds_fits<FMT, SELF>(kMaxPanels, true)) {
+    if (mm_lds_fits<FMT, SELF>(g.ppg, one)) {
+      if (one)
+        hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF, Epi::kOneTile, true>), grid, block, 0, stream, w, x16, batch, epi);
+      else
+        hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF, false, mm_lds_fits<FMT, SELF>(kMaxPanels, false)>), grid, block, 0,
+                           stream, w, x16, batch, epi);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF>), dim3(g.grid, g.groups), dim3(64u * g.ppg), 0, stream, w, x16, batch,
-                     epi);
+  if (one)
+    hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF, Epi::kOneTile>), grid, block, 0, stream, w, x16, batch, epi);
+  else
+    hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF>), grid, block, 0, stream, w, x16, batch, epi);
   return hipGetLastError();
 }
 

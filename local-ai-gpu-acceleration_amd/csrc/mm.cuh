@@ -285,6 +285,101 @@ __device__ __forceinline__ void mm_block_scale(const MmRaw& r, float& d, float& 
 
 // ---- the kernel ----------------------------------------------------------------------
 
+// ---- weights through LDS ------------------------------------------------------------
+//
+// A field load of mm_load touches 16 rows with 8 to 16 bytes a lane, and the L1
+// looks up a tag for about every lane: at the 8B gate_up the tags were busy 92 %
+// of the launch (TCP_TOTAL_CACHE_ACCESSES 52.7k per CU in 57k cycles), the VALU
+// 46 %, the LDS 26 %. Where a workgroup's row segment is a whole number of 16-byte
+// pieces (mm_lds_fits), it therefore copies each tile's 16 row segments to LDS
+// with whole-line loads, kMmPieces 16-byte pieces a thread, and the lanes read
+// their fields there. A row segment's image: its payload blocks, then (Q4_K
+// split-native) its heads, then 16 bytes of padding that spread the rows over the
+// banks.
+template <int FMT>
+constexpr std::uint32_t mm_row_bytes() {  // image bytes of one panel (512 columns)
+  return kPanelBlocks * (FmtBytes<FMT>::payload + FmtBytes<FMT>::meta);
+}
+template <int FMT>
+constexpr std::uint32_t mm_row_stride() { return kMaxPanels * mm_row_bytes<FMT>() + 16u; }
+// Pieces a thread copies: 16 rows of PB payload (or head) blocks per wave.
+template <int FMT>
+constexpr std::uint32_t mm_pieces() {
+  return (kPanelBlocks * FmtBytes<FMT>::payload + 63u) / 64u;
+}
+template <int FMT>
+constexpr std::uint32_t mm_head_pieces() {
+  return FmtBytes<FMT>::meta > 0u ? (kPanelBlocks * FmtBytes<FMT>::meta + 63u) / 64u : 0u;
+}
+// Whether workgroups of `waves` panels (one: of a single tile each) take the LDS
+// path: their segments start and end on 16-byte pieces of the stream (IQ blocks of
+// 82 and 110 bytes: 16 of them), and they fill a CU as one workgroup, as the field
+// loads' kernel does (smaller workgroups rely on several a CU, which the tiles'
+// LDS would not hold). Within that the faster one is taken, us of the field loads
+// / of LDS, batch 8, cold weights:
+//  * IQ: IQ2_S 28672x4096 23.5 / 20.0, 4096x4096 8.1 / 6.3; IQ3_S 27.6 / 23.6, 8.8
+//    / 6.7; with self-staging 14336x4096 19.4 / 17.6 and 21.7 / 19.8;
+//  * K-quants, whose field loads are whole 16 bytes a lane, gain less and lose the
+//    lines' early start behind self-staging (Q4_K 4096x14336 18.5 / 19.6, Q5_K 20.1
+//    / 21.2): not there; Q5_K 28672x4096 26.1 / 25.0 and the 8B LM head 94.9 / 82.7;
+//    Q4_K only as single tiles (4096x4096 8.3 / 6.5; 28672x4096 21.1 / 21.6).
+template <int FMT, bool SELF>
+constexpr bool mm_lds_fits(std::uint32_t waves, bool one) {
+  if (fmt_is_iq(FMT)) return waves == kMaxPanels;
+  return !SELF && waves >= kMaxPanels - 1u && (FMT == RTXLLM_FMT_Q5K || one);
+}
+
+// A lane's fields of block b of the wave's panel, from the row image: `p` the
+// block's payload bytes, `h` its head. IQ blocks are 2-byte aligned: the first of
+// a panel starts on a dword and has its fields 2 bytes off, the second the other
+// way round, so fields are read as whole dwords and shifted where they straddle.
+template <int FMT, int B>
+__device__ __forceinline__ void mm_lds_fields(const std::uint8_t* p, const std::uint8_t* h, std::uint32_t q,
+                                              MmRaw& r) {
+  auto dw = [](const std::uint8_t* a) { return *reinterpret_cast<const std::uint32_t*>(a); };
+  if constexpr (fmt_is_iq(FMT)) {
+    constexpr bool k2 = FMT == RTXLLM_FMT_IQ2S;
+    constexpr int QW = k2 ? 2 : 4;  // words of grid indices; two of signs
+    const std::uint8_t* qs = p + 2u + 4u * QW * q;
+    const std::uint8_t* sg = p + (k2 ? 34u : 74u) + 8u * q;
+    if constexpr (B % 2 == 0) {
+      std::uint32_t w[QW + 1], v[3];
+#pragma unroll
+      for (int i = 0; i <= QW; ++i) w[i] = dw(qs - 2 + 4 * i);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) v[i] = dw(sg - 2 + 4 * i);
+#pragma unroll
+      for (int i = 0; i < QW; ++i) r.a[i] = __builtin_amdgcn_alignbyte(w[i + 1], w[i], 2u);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) r.a[QW + i] = __builtin_amdgcn_alignbyte(v[i + 1], v[i], 2u);
+    } else {
+#pragma unroll
+      for (int i = 0; i < QW; ++i) r.a[i] = dw(qs + 4 * i);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) r.a[QW + i] = dw(sg + 4 * i);
+    }
+    r.s[0] = *reinterpret_cast<const std::uint16_t*>(p);
+    r.s[1] = *reinterpret_cast<const std::uint16_t*>(p + 66u + 2u * q);
+    if constexpr (k2)
+      r.s[2] = *reinterpret_cast<const std::uint16_t*>(p + 74u + 2u * q);
+    else
+      r.s8 = p[106u + q];
+  } else {
+    auto quad = [](const std::uint8_t* a, std::uint32_t* o) {
+      const uint4 t = *reinterpret_cast<const uint4*>(a);
+      o[0] = t.x, o[1] = t.y, o[2] = t.z, o[3] = t.w;
+    };
+    const std::uint8_t* qs = p + (FMT == RTXLLM_FMT_Q5K ? 48u : FMT == RTXLLM_FMT_Q4K_RAW ? 16u : 0u) + 32u * q;
+    quad(qs, r.a);
+    quad(qs + 16, r.a + 4);
+    if constexpr (FMT == RTXLLM_FMT_Q5K) {
+      quad(p + 16, r.b);
+      quad(p + 32, r.b + 4);
+    }
+    quad(FMT == RTXLLM_FMT_Q4K_SPLIT_NATIVE ? h : p, r.h);
+  }
+}
+
 // f(integral_constant<int, I>) for I = 0 .. N - 1, unrolled at compile time.
 template <int N, int I = 0, class F>
 __device__ __forceinline__ void static_for(F&& f) {
@@ -331,7 +426,10 @@ struct MmStore {
 // 7.8 us. With more tiles the re-reads stay: a tail without them for every
 // remainder, run once a launch, cost more in code than it saved (gate_up 21.9
 // -> 22.6 us).
-template <int FMT, class Epi, bool SELF = false, bool ONE = false>
+// LDSW: the weights go through LDS (above): tile t + 2 is requested into registers
+// while tile t is computed from one LDS buffer and tile t + 1 is written to the
+// other ahead of the tile's barrier.
+template <int FMT, class Epi, bool SELF = false, bool ONE = false, bool LDSW = false>
 __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const void* __restrict__ x16,
                                                              std::uint32_t batch, Epi epi) {
   // per-panel partial C of a tile, double buffered by tile parity
@@ -467,9 +565,51 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
   }
   constexpr int NB = mm_ring<FMT>();
   static_assert(NB >= PB, "a whole tile in the ring");
-  MmRaw ring[NB];
+  MmRaw ring[LDSW ? 1 : NB];
+  // LDSW: the thread's pieces (row of the tile, byte within the row segment, byte
+  // of the image), the same for every tile; pieces past the last one repeat it.
+  constexpr std::uint32_t KP = mm_pieces<FMT>(), KH = mm_head_pieces<FMT>(), RS = mm_row_stride<FMT>();
+  __shared__ uint4 wbuf[LDSW ? (ONE ? 1 : 2) : 1][LDSW ? 16u * RS / 16u : 1u];
+  std::uint32_t prow_of[KP + KH], pcol_of[KP + KH], pdst_of[KP + KH];
+  uint4 st[2][KP + KH];
+  const std::uint32_t nt = 64u * nw;
+  if constexpr (LDSW) {
+    const std::uint32_t pr = nw * PB * FmtBytes<FMT>::payload / 16u;  // payload pieces a row
+    const std::uint32_t hr = nw * PB * FmtBytes<FMT>::meta / 16u;     // head pieces a row
 #pragma unroll
-  for (int j = 0; j < (ONE ? PB : NB - 1); ++j) load_unit(static_cast<std::uint32_t>(j), ring[j]);
+    for (std::uint32_t j = 0; j < KP + KH; ++j) {
+      const bool head = j >= KP;
+      const std::uint32_t per = head ? hr : pr, count = 16u * per;
+      std::uint32_t i = threadIdx.x + (head ? j - KP : j) * nt;
+      i = i < count ? i : count - 1u;
+      const std::uint32_t row = i / per, piece = i - row * per;
+      prow_of[j] = row;
+      pcol_of[j] = 16u * piece + PB * nw * blockIdx.y * (head ? FmtBytes<FMT>::meta : FmtBytes<FMT>::payload);
+      pdst_of[j] = row * (RS / 16u) + piece + (head ? pr : 0u);
+    }
+  }
+  auto load_pieces = [&](std::uint32_t t, uint4 (&v)[KP + KH]) {  // tile number t of this workgroup
+    t = t < rounds ? t : rounds - 1u;
+    const std::uint32_t row0 = __builtin_amdgcn_readfirstlane((blockIdx.x + t * gridDim.x) * 16u);
+#pragma unroll
+    for (std::uint32_t j = 0; j < KP + KH; ++j) {
+      const std::uint32_t r = min(prow_of[j], rows - 1u - row0);  // rows past the last: read it again, not stored
+      const u32x4 x = j < KP ? bld_u128<0>(rsp, r * prow + pcol_of[j], row0 * prow)
+                             : bld_u128<0>(rsm, r * mrow + pcol_of[j], row0 * mrow);
+      v[j] = make_uint4(x.x, x.y, x.z, x.w);
+    }
+  };
+  auto write_pieces = [&](const uint4 (&v)[KP + KH], uint4* dst) {
+#pragma unroll
+    for (std::uint32_t j = 0; j < KP + KH; ++j) dst[pdst_of[j]] = v[j];
+  };
+  if constexpr (LDSW) {
+    load_pieces(0u, st[0]);
+    if constexpr (!ONE) load_pieces(1u, st[1]);
+  } else {
+#pragma unroll
+    for (int j = 0; j < (ONE ? PB : NB - 1); ++j) load_unit(static_cast<std::uint32_t>(j), ring[j]);
+  }
   if constexpr (!SELF) {
     __builtin_amdgcn_sched_barrier(0);  // the ring's loads ahead of the later blocks' operands
     const uint4* xb = reinterpret_cast<const uint4*>(x16) + PB * panel * 8u * 64u + lane;
@@ -479,8 +619,11 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
       for (int j = 0; j < 8; ++j) B[b][j] = xb[(8u * b + j) * 64u];
     __builtin_amdgcn_sched_barrier(0);
   }
+  if constexpr (LDSW) write_pieces(st[0], wbuf[0]);
   if constexpr (fmt_is_iq(FMT))
     lds_grid_commit(mm_lds<FMT>(), grid_stage, mm_image<FMT>(), threadIdx.x, blockDim.x);
+  else if constexpr (LDSW)
+    __syncthreads();
   tl_stamp(kTlR, tl_slot + 1u);
   float t_post = 1.0f;
   if constexpr (!SELF) {
@@ -529,12 +672,13 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
     __syncthreads();
     for (std::uint32_t e = threadIdx.x; e < 256u; e += 64u * nw) {  // whole waves
       float v = 0.0f;
-      if constexpr (fmt_is_iq(FMT)) {
+      if constexpr (FMT != RTXLLM_FMT_Q5K) {
         for (std::uint32_t k = 0; k < nw; ++k) v += red[round & 1u][k][e];
       } else {
         // every panel's read in flight, added in the same order (the LM head of
-        // the 8B batch-8 step 96.5 -> 94.6 us; in the IQ kernels, whose LDS serves
-        // the codebook lookups, it cost gate_up 4 %)
+        // the 8B batch-8 step 96.5 -> 94.6 us; not the others: in the IQ kernels,
+        // whose LDS serves the codebook lookups, it cost gate_up 4 %, and Q4_K
+        // 28672x4096 1 %)
         float r[kMaxPanels];
 #pragma unroll
         for (std::uint32_t k = 0; k < kMaxPanels; ++k) r[k] = red[round & 1u][k < nw ? k : nw - 1u][e];
@@ -550,29 +694,63 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
     tl_stamp(kTlR, tl_slot + 3u + (round < 11u ? round : 11u));
   };
 
-  // unit u sits in ring slot u % NB; PERIOD units bring both the slot and the
-  // block within the panel back. The main loop's body runs whole (no exit
-  // inside it, so the waits on the ring stay exact counts); the tail runs what
-  // is left.
-  constexpr int PERIOD = NB % PB == 0 ? NB : PB * NB;
-  auto step = [&](std::uint32_t u, auto jc) {
-    constexpr int j = decltype(jc)::value;
-    if constexpr (!ONE) {
-      load_unit(u + NB - 1u, ring[(j + NB - 1) % NB]);
-      __builtin_amdgcn_sched_barrier(0);  // the prefetch is issued before this unit's work
+  if constexpr (LDSW) {
+    // tile t (buffer BUF = t % 2): request tile t + 2 into the registers that
+    // held tile t, compute tile t, write tile t + 1 (requested a round ago), and
+    // meet at the tile's barrier
+    auto tile = [&](std::uint32_t t, auto bufc) {
+      constexpr int BUF = decltype(bufc)::value;
+      if constexpr (!ONE) {
+        load_pieces(t + 2u, st[BUF]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      const std::uint8_t* image = reinterpret_cast<const std::uint8_t*>(wbuf[ONE ? 0 : BUF]) + r16 * RS;
+      static_for<PB>([&](auto bc) {
+        constexpr std::uint32_t b = decltype(bc)::value;
+        MmRaw raw;
+        mm_lds_fields<FMT, decltype(bc)::value>(
+            image + (wave * PB + b) * FmtBytes<FMT>::payload,
+            image + nw * PB * FmtBytes<FMT>::payload + (wave * PB + b) * FmtBytes<FMT>::meta, q, raw);
+        finish_unit(b, raw);
+      });
+      if constexpr (!ONE) write_pieces(st[1 - BUF], wbuf[1 - BUF]);
+      tile_end(t);
+    };
+    if constexpr (ONE) {
+      tile(0u, std::integral_constant<int, 0>{});
+    } else {
+      for (std::uint32_t t = 0;;) {
+        tile(t, std::integral_constant<int, 0>{});
+        if (++t >= rounds) break;
+        tile(t, std::integral_constant<int, 1>{});
+        if (++t >= rounds) break;
+      }
     }
-    finish_unit(u, ring[j % NB]);
-    if constexpr (j % PB == PB - 1) tile_end(u / PB);
-  };
-  if constexpr (ONE) {
-    static_for<PB>([&](auto jc) { step(decltype(jc)::value, jc); });
   } else {
-    std::uint32_t u0 = 0;
-    for (; u0 + PERIOD <= units; u0 += PERIOD)
-      static_for<PERIOD>([&](auto jc) { step(u0 + decltype(jc)::value, jc); });
-    static_for<PERIOD>([&](auto jc) {
-      if (u0 + decltype(jc)::value < units) step(u0 + decltype(jc)::value, jc);
-    });
+    // unit u sits in ring slot u % NB; PERIOD units bring both the slot and the
+    // block within the panel back. The main loop's body runs whole (no exit
+    // inside it, so the waits on the ring stay exact counts); the tail runs what
+    // is left.
+    constexpr int PERIOD = NB % PB == 0 ? NB : PB * NB;
+    auto step = [&](std::uint32_t u, auto jc) {
+      constexpr int j = decltype(jc)::value;
+      if constexpr (!ONE) {
+        load_unit(u + NB - 1u, ring[(j + NB - 1) % NB]);
+        __builtin_amdgcn_sched_barrier(0);  // the prefetch is issued before this unit's work
+      }
+      finish_unit(u, ring[j % NB]);
+      if constexpr (j % PB == PB - 1) tile_end(u / PB);
+    };
+    if constexpr (ONE) {
+      static_for<PB>([&](auto jc) { step(decltype(jc)::value, jc); });
+    } else {
+      std::uint32_t u0 = 0;
+      for (; u0 + PERIOD <= units; u0 += PERIOD)
+        static_for<PERIOD>([&](auto jc) { step(u0 + decltype(jc)::value, jc); });
+      static_for<PERIOD>([&](auto jc) {
+        if (u0 + decltype(jc)::value < units) step(u0 + decltype(jc)::value, jc);
+      });
+    }
   }
   epi.finish(wave, lane, nw);
   tl_stamp(kTlR, tl_slot + 15u);

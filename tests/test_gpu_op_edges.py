@@ -250,3 +250,26 @@ def test_matvec_shared_staging_equals_staged_input(fmt, rows, cols):
             xd = at_offset(x, off)
             assert lib().rtxllm_matvec(fmt, P(w.payload), P(w.meta), P(xd), P(y), rows, cols, ops.stream()) == 0
             assert np.array_equal(y.cpu().numpy().view(np.uint32), ref.view(np.uint32)), (bad, off)
+
+
+@pytest.mark.parametrize("fmt", [F.Q4K_RAW, F.Q4K_SPLIT_NATIVE, F.Q5K, F.IQ2S, F.IQ3S], ids=lambda f: F.NAMES[f])
+@pytest.mark.parametrize("rows", [1, 100, 16400])
+@pytest.mark.parametrize("wide", [3584, 4096, 8192])
+def test_batch_weights_through_lds_equal_field_loads(fmt, rows, wide):
+    """Workgroups of seven or eight panels copy their weights through LDS (or, by the
+    rule, do not), smaller ones read fields: with x zero past the first 2048
+    columns the wide matrix gives the bits of its left 2048 columns."""
+    batch, left = 3, 2048
+    pack = packs.make_pack(fmt, rows, wide, seed=60 + fmt)
+    pb, mb, nb = F.PAYLOAD_BYTES[fmt], F.META_BYTES.get(fmt, 0), wide // 256
+
+    def part(a, width):
+        return np.ascontiguousarray(a.reshape(rows, nb, width)[:, :left // 256]).reshape(-1)
+
+    narrow = packs.Pack(fmt, rows, left, part(pack.payload, pb), None if pack.meta is None else part(pack.meta, mb))
+    x = np.zeros((batch, wide), np.float32)
+    x[:, :left] = packs.normal_f32(5, batch * left).reshape(batch, left)
+    y = ops.matvec_batch(ops.DevicePack(pack), ops.stage_batch(ops.to_dev(x)), batch).cpu().numpy()
+    xs = np.ascontiguousarray(x[:, :left])
+    ref = ops.matvec_batch(ops.DevicePack(narrow), ops.stage_batch(ops.to_dev(xs)), batch).cpu().numpy()
+    assert np.array_equal(y, ref)
