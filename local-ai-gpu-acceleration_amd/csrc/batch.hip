@@ -249,17 +249,17 @@ struct MmLogits {
 
 // Workgroups of mm_kernel<FMT, Epi> of `threads` threads resident per CU (0 if
 // the query fails), cached per size.
-template <int FMT, class Epi, bool SELF = false>
+// ONE: of the single-tile kernel.
+template <int FMT, class Epi, bool SELF = false, bool ONE = false>
 int mm_resident(std::uint32_t threads) {
   static int cache[kMaxPanels + 1] = {};
   const std::uint32_t w = threads / 64u;
   if (w == 0u || w > kMaxPanels) return 0;
   if (cache[w] == 0) {
     int n = 0;
-    // the kernel of a persistent grid (a single-tile grid takes its geometry)
-    const void* f = reinterpret_cast<const void*>(&mm_kernel<FMT, Epi, SELF>);
-    if constexpr (mm_lds_fits<FMT, SELF>(kMaxPanels, false))
-      if (mm_lds_fits<FMT, SELF>(w, false)) f = reinterpret_cast<const void*>(&mm_kernel<FMT, Epi, SELF, false, true>);
+    const void* f = reinterpret_cast<const void*>(&mm_kernel<FMT, Epi, SELF, ONE>);
+    if constexpr (mm_lds_fits<FMT, SELF>(kMaxPanels, ONE))
+      if (mm_lds_fits<FMT, SELF>(w, ONE)) f = reinterpret_cast<const void*>(&mm_kernel<FMT, Epi, SELF, ONE, true>);
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, f, static_cast<int>(threads), 0) != hipSuccess || n <= 0)
       return 0;
     cache[w] = n;
@@ -310,9 +310,21 @@ hipError_t launch_mm_epi(const QTensor& w, const void* x16, std::uint32_t batch,
   const std::uint64_t blocks = static_cast<std::uint64_t>(w.rows) * (w.cols / 256u);
   if (blocks * FmtBytes<FMT>::payload > 0xFFFFFFFFull || blocks * FmtBytes<FMT>::meta > 0xFFFFFFFFull)
     return hipErrorInvalidValue;
+  const std::uint32_t tiles = (w.rows + 15u) / 16u;
+  bool one = Epi::kOneTile && g.grid == tiles;  // every tile resident
+  if constexpr (Epi::kOneTile && mm_lds_fits<FMT, SELF>(kMaxPanels, true)) {
+    // Through LDS the single-tile kernel is small enough for several workgroups a
+    // CU: where all tiles are then resident at once (up to two a CU) it beats two
+    // rounds of the persistent grid, whose second waits for the first (the 8B
+    // qkv, 384 tiles: 10.9 -> 10.4 us; the batch-8 step 2776 -> 2750).
+    if (!one && mm_lds_fits<FMT, SELF>(g.ppg, true) && g.groups == 1u &&
+        tiles <= static_cast<std::uint32_t>(std::min(2, mm_resident<FMT, Epi, SELF, true>(64u * g.ppg)) * num_cus())) {
+      one = true;
+      g.grid = tiles;
+    }
+  }
   if (geom != nullptr) *geom = g;
   const dim3 grid(g.grid, g.groups), block(64u * g.ppg);
-  const bool one = Epi::kOneTile && g.grid == (w.rows + 15u) / 16u;  // every tile resident
   if constexpr (mm_lds_fits<FMT, SELF>(kMaxPanels, true)) {
     if (mm_lds_fits<FMT, SELF>(g.ppg, one)) {
       if (one)
