@@ -503,7 +503,7 @@ hipError_t matvec_batch(int format, const uint8_t* payload, const uint8_t* meta,
                                                     batch, out, stream)
                              : launch_mm_batch(format, payload, meta, rows, cols, x, batch, out, stream);
   if (st != hipSuccess || groups == 1u) return st;
-  hipLaunchKernelGGL(mm_reduce_kernel, dim3(static_cast<unsigned>((n + 255u) / 256u)), dim3(256), 0, stream,
+  hipLaunchKernelGGL(mm_reduce_kernel, dim3(static_cast<unsigned>((n + 255u) / 256u)), dim3(64), 0, stream,
                      static_cast<const float*>(workspace), groups, static_cast<std::uint32_t>(n), y);
   return hipGetLastError();
 }

@@ -756,14 +756,35 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
   tl_stamp(kTlR, tl_slot + 15u);
 }
 
-// y[s][r] = sum over panel groups of partial[pg][s][r].
-__global__ void mm_reduce_kernel(const float* __restrict__ partial, std::uint32_t groups, std::uint32_t n,
-                                 float* __restrict__ y) {
-  const std::uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+// y[i] = sum over panel groups of partial[pg][i], in group order, four values a
+// thread (n = batch x rows need not be a multiple of four). All latency: up to
+// eight groups' reads in flight, where a loop over the groups waited for each
+// (batch 8, Q4_K 4096 x 14336, four groups: 17.9 -> 17.2 us with the matvec).
+__global__ __launch_bounds__(64) void mm_reduce_kernel(const float* __restrict__ partial, std::uint32_t groups,
+                                                       std::uint32_t n, float* __restrict__ y) {
+  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+  const std::uint32_t i = 4u * (blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= n) return;
-  float s = 0.0f;
-  for (std::uint32_t g = 0; g < groups; ++g) s += partial[static_cast<std::size_t>(g) * n + i];
-  y[i] = s;
+  if (n - i < 4u) {
+    for (std::uint32_t k = i; k < n; ++k) {
+      float s = 0.0f;
+      for (std::uint32_t g = 0; g < groups; ++g) s += partial[static_cast<std::size_t>(g) * n + k];
+      y[k] = s;
+    }
+    return;
+  }
+  f32x4_any s = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (std::uint32_t g0 = 0; g0 < groups; g0 += 8u) {
+    f32x4_any v[8];
+#pragma unroll
+    for (std::uint32_t j = 0; j < 8u; ++j) {
+      const std::uint32_t g = g0 + j < groups ? g0 + j : groups - 1u;
+      v[j] = *reinterpret_cast<const f32x4_any*>(partial + static_cast<std::size_t>(g) * n + i);
+    }
+#pragma unroll
+    for (std::uint32_t j = 0; j < 8u; ++j) s = g0 + j < groups ? s + v[j] : s;
+  }
+  *reinterpret_cast<f32x4_any*>(y + i) = s;
 }
 
 }  // namespace rtxllm

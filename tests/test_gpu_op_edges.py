@@ -273,3 +273,17 @@ def test_batch_weights_through_lds_equal_field_loads(fmt, rows, wide):
     xs = np.ascontiguousarray(x[:, :left])
     ref = ops.matvec_batch(ops.DevicePack(narrow), ops.stage_batch(ops.to_dev(xs)), batch).cpu().numpy()
     assert np.array_equal(y, ref)
+
+
+@pytest.mark.parametrize("rows,batch", [(1, 1), (3, 1), (5, 3), (64, 8), (1023, 7)])
+@pytest.mark.parametrize("cols", [4608, 5632, 10240])
+def test_batch_panel_groups_are_added(orc, rows, batch, cols):
+    """Three, eleven and four panel groups (fewer and more than the reduction
+    reads at once), rows x batch with every remainder of four."""
+    pack = packs.make_pack(F.Q4K_SPLIT_NATIVE, rows, cols, seed=70)
+    xs = packs.normal_f32(rows, batch * cols).reshape(batch, cols)
+    y = ops.matvec_batch(ops.DevicePack(pack), ops.stage_batch(ops.to_dev(xs)), batch).cpu().numpy()
+    for s in range(batch):
+        ref = orc.matvec_f32(F.Q4K_SPLIT_NATIVE, pack.payload, pack.meta, xs[s], rows, cols, 8)
+        # the fp32 sequential oracle's own error at these widths
+        assert float(np.max(np.abs(y[s] - ref))) <= 1e-4 * float(np.max(np.abs(ref)))
