@@ -217,8 +217,9 @@ hipError_t rtxllm_launch_q4k_matvec_decode_split_native_vec4x4(const uint8_t* q4
 hipError_t rtxllm_dequant_f32(int format, const uint8_t* payload, const uint8_t* meta, uint32_t rows,
                               uint32_t cols, float* out, hipStream_t stream);
 
-/* y[rows] = W x (batch 1), no side effects. x is fp32; each wave stages the
- * columns it owns itself (the rtxllm_stage_activation rule). */
+/* y[rows] = W x (batch 1), no side effects. x is fp32; the kernel stages it
+ * itself, a wave its own columns or a workgroup all of them (the
+ * rtxllm_stage_activation rule, the same bits either way). */
 hipError_t rtxllm_matvec(int format, const uint8_t* payload, const uint8_t* meta, const float* x, float* y,
                          uint32_t rows, uint32_t cols, hipStream_t stream);
 
