@@ -220,7 +220,9 @@ extern "C" hipError_t rtxllm_rmsnorm_w(const float* x, const float* weight, uint
                                        float* out, hipStream_t stream) {
   if (x == nullptr || out == nullptr || n == 0u || count == 0u || count > 65535u * 1024u || !(eps >= 0.0f))
     return hipErrorInvalidValue;
-  const bool vec = (n % 4u) == 0u && n <= 16384u &&
+  // (a launch holds fewer than 2^32 threads: more than 2^22 - 1 vectors wider than
+  // 4096 stay with the 256-thread kernel)
+  const bool vec = (n % 4u) == 0u && n <= 16384u && (n <= 4096u || count < (1u << 22)) &&
                    ((reinterpret_cast<std::uintptr_t>(x) | reinterpret_cast<std::uintptr_t>(weight) |
                      reinterpret_cast<std::uintptr_t>(out)) % 16u) == 0u;
   // Few vectors leave the chip idle and the one workgroup's latency is the time:
