@@ -108,29 +108,51 @@ inline int mv_resident(std::uint32_t block_threads) {
 
 // Row groups per workgroup of the shared self-staging kernel (0: the kernel whose
 // waves stage their own columns). Same results bit for bit, so the line is drawn
-// by time alone (fp32 x, cold weights, us of each without / with sharing):
-//  * IQ formats, up to 8 waves a workgroup: IQ2_S 8192x2048 7.7 / 5.5, 14336x4096
-//    14.1 / 9.8, 4096x8192 11.8 / 8.6; IQ3_S 7.2 / 6.0, 13.2 / 11.1, 10.2 / 9.3;
-//  * K-quants only where one wave holds a row (Q5_K 8192x2048 5.7 / 5.5), Q4_K up
-//    to 1024 columns (30001x1024 9.6 / 9.1; 8192x2048 5.1 / 5.2); with two waves
-//    a row the barrier costs more (Q4_K 4096x4096 5.2 / 6.0);
+// by time alone, over 256 to 64000 rows and 256 to 8192 columns (fp32 x, cold
+// weights, us of each without / with sharing). ks: waves a row; fill: whole
+// 4-row tiles a CU. One row group a workgroup stages all of x as its wave would
+// alone, and passes it through LDS (Q5_K 2000x2048 4.1 / 5.4), and three or six
+// leave a last round of workgroups on part of the CUs (IQ3_S 3600x2560 with three
+// 6.6 / 7.1, with four 5.6).
+//  * IQ formats, a wave a row: four groups (IQ2_S 256x2048 4.9 / 3.8, 8192x2048 7.5
+//    / 5.2; IQ3_S 3000x2048 5.1 / 4.7), eight from 16 tiles a CU on (IQ2_S 22000x768:
+//    without 13.0, four 8.2, eight 7.8);
+//  * two waves a row: four groups from two tiles a CU on (IQ2_S 14336x4096 14.6 /
+//    10.8, IQ3_S 4096x4096 7.4 / 6.6); with fewer they leave CUs idle (IQ3_S
+//    2000x4096 5.3 / 5.9);
+//  * three or four: two groups, IQ2_S from two tiles a CU on (4096x8192 12.6 / 9.1),
+//    in units with three waves up to nine (8192x5632 15.0 / 13.5, 14336x5632 18.4 /
+//    19.0); IQ3_S with four waves from three tiles on (4096x8192 11.0 / 10.2,
+//    3000x8192 9.3 / 9.8), with three between four and nine and not in units
+//    (6000x5120 11.6 / 11.1, 3000x5120 7.9 / 8.3, 14336x6144 17.5 / 18.4, in units
+//    7000x6144 12.8 / 16.2);
+//  * K-quants only where one wave holds a row. Up to 1024 columns and below two
+//    tiles a CU, two groups, or one where a workgroup each then fills no more than
+//    the CUs and x is short (Q4_K 1000x512 3.5 / 3.1, 1000x1024 3.5 / 3.2). Else
+//    Q5_K four (2000x2048 4.1 / 3.8, 14336x1024 8.1 / 7.4), Q4_K, up to 1024
+//    columns, four from five tiles on (12000x1024 6.0 / 5.5) and none before
+//    (3000x1024 3.5 / 3.7 with four, 4.4 with two);
 //  * not from four rounds a row group on, where the staging is paid off anyway
-//    and the row groups of a workgroup run in step (IQ3_S 64000x2560 29.3 / 31.3);
-//  * no more row groups than keep a workgroup on every CU (IQ3_S 4096x1024 4.5 /
-//    4.8 with eight on half of the CUs, 4.1 with four), and none where that
-//    leaves several waves one row group to stage for (2000x8192 7.3 / 8.2).
+//    and the row groups of a workgroup run in step (IQ3_S 64000x2560 29.3 / 31.3).
 template <int FMT, bool SELF, class Epi>
 inline std::uint32_t mv_share_groups(std::uint32_t rows, std::uint32_t cols) {
   if constexpr (!SELF || EpiGroupRows<Epi>::value > 0u) return 0u;
   const std::uint32_t ks = (cols / 32u + 63u) / 64u, cus = static_cast<std::uint32_t>(num_cus());
-  const std::uint32_t tiles = (rows + Epi::kTile - 1u) / Epi::kTile;
-  const bool k_quant = ks == 1u && (FMT == RTXLLM_FMT_Q5K || cols <= 1024u);
-  const std::uint32_t most = fmt_is_iq(FMT) ? 8u / ks : (k_quant ? 4u : 0u);
+  const std::uint32_t tiles = (rows + Epi::kTile - 1u) / Epi::kTile, fill = tiles / cus;
   // 16 waves a CU resident: 16 / ks row groups
-  if (cols > kSelfShareCols || most == 0u || static_cast<std::uint64_t>(tiles) * ks > 4ull * 16ull * cus) return 0u;
-  const std::uint32_t fill = tiles / cus < 1u ? 1u : tiles / cus;
-  const std::uint32_t groups = fill < most ? fill : most;
-  return groups == 1u && ks > 1u ? 0u : groups;
+  if (cols > kSelfShareCols || static_cast<std::uint64_t>(tiles) * ks > 4ull * 16ull * cus) return 0u;
+  if constexpr (!fmt_is_iq(FMT)) {
+    if (ks > 1u || (FMT != RTXLLM_FMT_Q5K && cols > 1024u)) return 0u;
+    if (cols <= 1024u && fill < 2u) return cols <= 512u && fill == 0u ? 1u : 2u;
+    return FMT == RTXLLM_FMT_Q5K || fill >= 5u ? 4u : 0u;
+  }
+  if (ks == 1u) return fill < 16u ? 4u : 8u;
+  if (ks == 2u) return fill < 2u ? 0u : 4u;
+  if constexpr (FMT == RTXLLM_FMT_IQ3S || FMT == RTXLLM_FMT_IQ3S_UNITS) {
+    if (ks == 4u) return fill < 3u ? 0u : 2u;
+    return FMT == RTXLLM_FMT_IQ3S && fill >= 4u && fill < 9u ? 2u : 0u;
+  }
+  return fill >= 2u && (FMT != RTXLLM_FMT_IQ2S_UNITS || ks == 4u || fill < 9u) ? 2u : 0u;
 }
 
 template <int FMT, bool SELF, class Epi>

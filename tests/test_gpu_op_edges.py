@@ -230,9 +230,10 @@ def test_rmsnorm_feedback_edges(rows, cols, offset):
 @pytest.mark.parametrize("fmt", [F.Q4K_SPLIT_NATIVE, F.Q4K_SPLIT_COMPACT, F.Q5K, F.IQ2S, F.IQ3S, F.IQ2S_UNITS,
                                  F.IQ3S_UNITS], ids=lambda f: F.NAMES[f])
 @pytest.mark.parametrize("rows,cols", [(1, 256), (1023, 512), (1030, 1024), (2049, 2048), (2055, 2304), (4097, 4096),
-                                       (8195, 4352), (2048, 8192), (2051, 8448), (4099, 8192), (70001, 256)])
+                                       (8195, 4352), (2048, 8192), (2051, 8448), (4099, 8192), (70001, 256),
+                                       (3001, 1024), (5401, 768), (17001, 512), (2055, 4608), (9301, 4608)])
 def test_matvec_shared_staging_equals_staged_input(fmt, rows, cols):
-    """One to eight row groups a workgroup share the staging of an fp32 x, or none
+    """One, two, four or eight row groups a workgroup share the staging of an fp32 x, or none
     do (widths, row counts and formats on both sides of the rule): always the
     bits of rtxllm_stage_activation + rtxllm_matvec_xq, x aligned or not, and a
     NaN or infinite value poisons as there."""
