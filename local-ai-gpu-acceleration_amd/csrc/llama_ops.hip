@@ -105,11 +105,11 @@ __device__ __forceinline__ float2 rope_cos_sin(std::uint32_t i, std::uint32_t he
   return make_float2(static_cast<float>(cos(angle)), static_cast<float>(sin(angle)));
 }
 
-// Workgroup (chunk of kRopePairs P pairs, vector r = blockIdx.y): the head_dim / 2
+// Workgroup (chunk of kOpThreads P pairs, vector r = blockIdx.y): the head_dim / 2
 // angles of the vector once, into LDS, then P pairs a thread, whose loads were
 // issued before. Against one double pow, cos and sin per pair of every head:
-// 256 vectors of 32 heads 8.3 -> 4.1 us, one vector 4.7 -> 2.9 us.
-constexpr std::uint32_t kRopeMaxHalf = 1024;  // head_dim / 2 at most, or one thread per pair (below)
+// 256 vectors of 32 heads of 128 8.0 -> 4.1 us (where it pays: rope_shared_pairs).
+constexpr std::uint32_t kRopeMaxHalf = 1024;  // head_dim / 2 at most
 template <std::uint32_t P>
 __global__ __launch_bounds__(kOpThreads) void rope_theta_kernel(float* __restrict__ vec, std::uint32_t pairs,
                                                                 std::uint32_t head_dim, double theta,
@@ -135,8 +135,8 @@ __global__ __launch_bounds__(kOpThreads) void rope_theta_kernel(float* __restric
   }
 }
 
-// Heads of more than 2 kRopeMaxHalf values: one thread per pair, its own angle.
-__global__ __launch_bounds__(kOpThreads) void rope_theta_wide_kernel(float* __restrict__ vec, std::uint32_t pairs,
+// One thread per pair, its own angle.
+__global__ __launch_bounds__(kOpThreads) void rope_theta_pair_kernel(float* __restrict__ vec, std::uint32_t pairs,
                                                                      std::uint32_t head_dim, double theta,
                                                                      const std::uint32_t* __restrict__ pos) {
   const std::uint32_t p = blockIdx.x * kOpThreads + threadIdx.x;
@@ -203,6 +203,25 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(const float
   if (threadIdx.x == 0u) index[blockIdx.x] = i;
 }
 
+// Pairs a thread of the shared-angle rotary kernel, or 0: one thread per pair. A
+// few double evaluations more or less don't show in a launch of 3 us: sharing pays
+// from where it saves one for every lane of the chip's 1024 SIMDs; short of that
+// its LDS pass and barrier cost 1 to 10 % (us of own / shared angles, heads x head_dim, vectors: 32x128
+// x256 8.0 / 4.1, x64 3.7 / 3.4, x32 3.0 / 3.1; 8x32 x64 3.0 / 3.3; 2x2048 x48
+// 3.6 / 7.7). Heads of more than 512 values, whose threads evaluate several
+// angles in turn, need half as much again (4x1024 x64 3.7 / 4.3, x128 5.1 /
+// 4.5). Vectors of up to 128 pairs leave most of a workgroup's threads idle
+// (1x256 x2048 5.2 / 6.6). Below 64 vectors one pair a thread spreads the loads
+// over more workgroups (32x128 x48: one 3.1, four 3.4).
+std::uint32_t rope_shared_pairs(std::uint32_t pairs, std::uint32_t half, std::uint32_t count) {
+  if (half > kRopeMaxHalf || pairs <= 128u) return 0u;
+  const std::uint32_t per = half > kOpThreads || count >= 64u ? 4u : 1u;
+  const std::uint64_t chunks = (pairs + kOpThreads * per - 1u) / (kOpThreads * per);
+  const std::uint64_t own = static_cast<std::uint64_t>(pairs) * count, shared = chunks * half * count;
+  constexpr std::uint64_t kLanes = 1024u * 64u;
+  return own > shared + (half > kOpThreads ? kLanes + kLanes / 2u : kLanes) ? per : 0u;
+}
+
 bool group_ok(std::uint32_t n_heads, std::uint32_t n_kv) {
   if (n_kv == 0u || n_heads == 0u || n_heads % n_kv != 0u) return false;
   const std::uint32_t g = n_heads / n_kv;
@@ -249,14 +268,12 @@ extern "C" hipError_t rtxllm_rope_theta(float* vec, uint32_t n_heads, uint32_t h
   const std::uint64_t pairs = static_cast<std::uint64_t>(n_heads) * head_dim / 2u;
   if (pairs > 0xFFFFFFFFull / 2u) return hipErrorInvalidValue;
   const std::uint32_t np = static_cast<std::uint32_t>(pairs);
-  // 1024 pairs a workgroup share one set of angles; few vectors keep small
-  // workgroups, so that their loads spread over the CUs
-  const std::uint32_t per = head_dim / 2u > kRopeMaxHalf || count < 64u ? 1u : 4u;
+  const std::uint32_t shared = rope_shared_pairs(np, head_dim / 2u, count), per = shared > 0u ? shared : 1u;
   const dim3 grid((np + kOpThreads * per - 1u) / (kOpThreads * per), count);
-  if (head_dim / 2u > kRopeMaxHalf)
-    hipLaunchKernelGGL(rope_theta_wide_kernel, grid, dim3(kOpThreads), 0, stream, vec, np, head_dim,
+  if (shared == 0u)
+    hipLaunchKernelGGL(rope_theta_pair_kernel, grid, dim3(kOpThreads), 0, stream, vec, np, head_dim,
                        static_cast<double>(theta), pos);
-  else if (per == 1u)
+  else if (shared == 1u)
     hipLaunchKernelGGL(rope_theta_kernel<1>, grid, dim3(kOpThreads), 0, stream, vec, np, head_dim,
                        static_cast<double>(theta), pos);
   else

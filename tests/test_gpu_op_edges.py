@@ -104,10 +104,12 @@ def test_rmsnorm_edges(n, count, offset):
 
 
 @pytest.mark.parametrize("heads,head_dim,count", [(1, 2, 1), (3, 6, 2), (5, 128, 63), (9, 128, 64), (2, 96, 70),
-                                                  (33, 64, 65), (1, 2048, 64), (1, 2050, 2), (2, 2050, 65)])
+                                                  (33, 64, 65), (1, 2048, 64), (1, 2050, 2), (2, 2050, 65),
+                                                  (33, 128, 48), (33, 64, 130), (9, 512, 64), (5, 1026, 128)])
 def test_rope_edges(heads, head_dim, count):
-    """One and four pairs a thread, remainders of both, the widest shared-angle
-    head and the one past it, against float64 rotation of the fp32 angle."""
+    """A thread per pair, shared angles with one and with four pairs a thread, the
+    remainders of each, and heads with more angles than a workgroup has threads,
+    against float64 rotation of the fp32 angle."""
     theta = 10000.0
     vec = packs.normal_f32(head_dim, count * heads * head_dim).reshape(count, heads, head_dim // 2, 2)
     pos = (np.arange(count, dtype=np.uint32) * 37 + 5).astype(np.uint32)
