@@ -672,18 +672,23 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
     __syncthreads();
     for (std::uint32_t e = threadIdx.x; e < 256u; e += 64u * nw) {  // whole waves
       float v = 0.0f;
-      if constexpr (FMT != RTXLLM_FMT_Q5K) {
+      if constexpr (FMT != RTXLLM_FMT_Q5K || SELF) {
         for (std::uint32_t k = 0; k < nw; ++k) v += red[round & 1u][k][e];
       } else {
         // every panel's read in flight, added in the same order (the LM head of
         // the 8B batch-8 step 96.5 -> 94.6 us; not the others: in the IQ kernels,
-        // whose LDS serves the codebook lookups, it cost gate_up 4 %, and Q4_K
-        // 28672x4096 1 %)
-        float r[kMaxPanels];
+        // whose LDS serves the codebook lookups, it cost gate_up 4 %, Q4_K
+        // 28672x4096 1 % and self-staging 2 %). A single panel has nothing to wait
+        // for: the eight clamped reads cost it 3 to 6 % (4096x512: 3.9 -> 4.2 us)
+        if (nw == 1u) {
+          v = red[round & 1u][0][e];
+        } else {
+          float r[kMaxPanels];
 #pragma unroll
-        for (std::uint32_t k = 0; k < kMaxPanels; ++k) r[k] = red[round & 1u][k < nw ? k : nw - 1u][e];
+          for (std::uint32_t k = 0; k < kMaxPanels; ++k) r[k] = red[round & 1u][k < nw ? k : nw - 1u][e];
 #pragma unroll
-        for (std::uint32_t k = 0; k < kMaxPanels; ++k) v = k < nw ? v + r[k] : v;
+          for (std::uint32_t k = 0; k < kMaxPanels; ++k) v = k < nw ? v + r[k] : v;
+        }
       }
       const float tot = v + __shfl_xor(v, 4, 64);  // column n ^ 1 is lane l ^ 1 = element e ^ 4
       const float y = tot * t_post;
