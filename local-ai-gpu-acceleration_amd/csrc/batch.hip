@@ -300,6 +300,14 @@ bool mm_geom(std::uint32_t rows, std::uint32_t cols, MmGeom& g) {
   return true;
 }
 
+// Whether a launch of `workgroups` takes its weights through LDS (mm_lds_fits; at
+// seven panels of Q5_K not past one workgroup a CU).
+template <int FMT, bool SELF>
+inline bool mm_takes_lds(std::uint32_t ppg, bool one, std::uint32_t workgroups) {
+  return mm_lds_fits<FMT, SELF>(ppg, one) &&
+         (FMT != RTXLLM_FMT_Q5K || ppg == kMaxPanels || workgroups <= static_cast<std::uint32_t>(num_cus()));
+}
+
 template <int FMT, bool SELF = false, class Epi>
 hipError_t launch_mm_epi(const QTensor& w, const void* x16, std::uint32_t batch, const Epi& epi, bool one_group,
                          MmGeom* geom, hipStream_t stream) {
@@ -317,7 +325,7 @@ hipError_t launch_mm_epi(const QTensor& w, const void* x16, std::uint32_t batch,
     // CU: where all tiles are then resident at once (up to two a CU) it beats two
     // rounds of the persistent grid, whose second waits for the first (the 8B
     // qkv, 384 tiles: 10.9 -> 10.4 us; the batch-8 step 2776 -> 2750).
-    if (!one && mm_lds_fits<FMT, SELF>(g.ppg, true) && g.groups == 1u &&
+    if (!one && mm_takes_lds<FMT, SELF>(g.ppg, true, tiles) && g.groups == 1u &&
         tiles <= static_cast<std::uint32_t>(std::min(2, mm_resident<FMT, Epi, SELF, true>(64u * g.ppg)) * num_cus())) {
       one = true;
       g.grid = tiles;
@@ -326,7 +334,7 @@ hipError_t launch_mm_epi(const QTensor& w, const void* x16, std::uint32_t batch,
   if (geom != nullptr) *geom = g;
   const dim3 grid(g.grid, g.groups), block(64u * g.ppg);
   if constexpr (mm_lds_fits<FMT, SELF>(kMaxPanels, true)) {
-    if (mm_lds_fits<FMT, SELF>(g.ppg, one)) {
+    if (mm_takes_lds<FMT, SELF>(g.ppg, one, g.grid * g.groups)) {
       if (one)
         hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF, Epi::kOneTile, true>), grid, block, 0, stream, w, x16, batch, epi);
       else

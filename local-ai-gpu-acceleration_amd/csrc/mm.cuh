@@ -321,12 +321,15 @@ constexpr std::uint32_t mm_head_pieces() {
 //    / 6.7; with self-staging 14336x4096 19.4 / 17.6 and 21.7 / 19.8;
 //  * K-quants, whose field loads are whole 16 bytes a lane, gain less and lose the
 //    lines' early start behind self-staging (Q4_K 4096x14336 18.5 / 19.6, Q5_K 20.1
-//    / 21.2): not there; Q5_K 28672x4096 26.1 / 25.0 and the 8B LM head 94.9 / 82.7;
-//    Q4_K only as single tiles (4096x4096 8.3 / 6.5; 28672x4096 21.1 / 21.6).
+//    / 21.2): not there. Eight panels of Q5_K 28672x4096 26.1 / 25.0 and the 8B LM
+//    head 94.9 / 82.7; seven lose (32000x3584 22.5 / 24.3, 11008x3584 12.1 / 13.3)
+//    but as single tiles, one a CU (4096x3584 7.3 / 6.9). Q4_K only as single tiles
+//    (4096x4096 8.3 / 6.5; 28672x4096 21.1 / 21.6).
 template <int FMT, bool SELF>
 constexpr bool mm_lds_fits(std::uint32_t waves, bool one) {
   if (fmt_is_iq(FMT)) return waves == kMaxPanels;
-  return !SELF && waves >= kMaxPanels - 1u && (FMT == RTXLLM_FMT_Q5K || one);
+  if (SELF || waves < kMaxPanels - 1u) return false;
+  return one || (FMT == RTXLLM_FMT_Q5K && waves == kMaxPanels);
 }
 
 // A lane's fields of block b of the wave's panel, from the row image: `p` the
