@@ -308,6 +308,33 @@ inline bool mm_takes_lds(std::uint32_t ppg, bool one, std::uint32_t workgroups) 
          (FMT != RTXLLM_FMT_Q5K || ppg == kMaxPanels || workgroups <= static_cast<std::uint32_t>(num_cus()));
 }
 
+// Whether workgroups of one tile that read fields take the single-tile kernel. It
+// requests the whole tile at once, so the codebook or the conversion of x waits
+// behind more loads than in the ring kernel, whose grid holds the same tiles: us of
+// ring / single tile at batch 8, by panels a workgroup.
+//  * staged x: always but Q5_K with four, one a CU (4096x2048 4.7 / 4.9);
+//  * self-staging IQ3_S: but four, one a CU, past six sequences (1000x2048 7.5 /
+//    7.7, of four 7.4 / 7.2; others 1000x512 6.2 / 5.9, 1000x3072 10.6 / 10.0,
+//    8192x2048 11.9 / 11.3);
+//  * self-staging IQ2_S: one, one a CU; from six; others with more than one a CU
+//    (1000x3072 10.4 / 9.9, 8192x2048 11.6 / 11.2; but 1000x2048 7.2 / 7.6,
+//    14336x512 8.3 / 8.7);
+//  * self-staging Q4_K raw: three, four and from seven; one and two past three a CU
+//    (8192x2048 10.7 / 9.7, 4096x4096 10.6 / 9.7, 32000x512 11.3 / 10.1; but
+//    4096x512 5.7 / 6.0, 4096x2560 8.8 / 9.1);
+//  * self-staging Q5_K and Q4_K split-native: never (Q5_K 4096x1024 6.0 / 6.3,
+//    4096x3072 9.4 / 9.7; Q4_K 4096x512 5.9 / 6.1, 500x5120 10.2 / 10.5 at batch 2).
+template <int FMT, bool SELF>
+inline bool mm_one_tile_pays(std::uint32_t ppg, std::uint32_t workgroups, std::uint32_t batch) {
+  const std::uint32_t cus = static_cast<std::uint32_t>(num_cus());
+  const bool shared_cu = workgroups > cus;
+  if (!SELF) return FMT != RTXLLM_FMT_Q5K || ppg != 4u || shared_cu;
+  if (FMT == RTXLLM_FMT_IQ3S) return ppg != 4u || shared_cu || batch <= 6u;
+  if (FMT == RTXLLM_FMT_IQ2S) return ppg == 1u ? !shared_cu : (ppg >= 6u || shared_cu);
+  if (FMT == RTXLLM_FMT_Q4K_RAW) return ppg <= 2u ? workgroups > 3u * cus : (ppg <= 4u || ppg >= 7u);
+  return false;
+}
+
 template <int FMT, bool SELF = false, class Epi>
 hipError_t launch_mm_epi(const QTensor& w, const void* x16, std::uint32_t batch, const Epi& epi, bool one_group,
                          MmGeom* geom, hipStream_t stream) {
@@ -343,7 +370,7 @@ hipError_t launch_mm_epi(const QTensor& w, const void* x16, std::uint32_t batch,
       return hipGetLastError();
     }
   }
-  if (one)
+  if (one && mm_one_tile_pays<FMT, SELF>(g.ppg, g.grid * g.groups, batch))
     hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF, Epi::kOneTile>), grid, block, 0, stream, w, x16, batch, epi);
   else
     hipLaunchKernelGGL((mm_kernel<FMT, Epi, SELF>), grid, block, 0, stream, w, x16, batch, epi);
