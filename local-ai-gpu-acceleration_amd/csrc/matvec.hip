@@ -45,34 +45,40 @@ bool pointers_ok(int fmt, const void* payload, const void* meta, const void* x, 
 // alignment (gfx950 stores unaligned 16-byte vectors).
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-// A wave expands kDequantBlocks consecutive blocks (out is the blocks in order:
-// 256 values each), lane l four values of each: 1 KB of whole lines per store.
-// The kernel is bound by its writes (fp32 out is 7 to 12 times the pack's
-// bytes): nontemporal, as nothing here reads them again. Q4_K 14336 x 4096:
-// 38.5 us, 6.95 TB/s of pack and output; one value per thread (the head decoded
-// 256 times a block, 4-byte stores) took 160.0 us.
-constexpr std::uint32_t kDequantBlocks = 4;
-template <int FMT>
+// A wave expands PER consecutive blocks (out is the blocks in order: 256 values
+// each), lane l four values of each: 1 KB of whole lines per store. The kernel is
+// bound by its writes (fp32 out is 7 to 12 times the pack's bytes). Q4_K 14336 x
+// 4096: 38.5 us, 6.95 TB/s of pack and output; one value per thread (the head
+// decoded 256 times a block, 4-byte stores) took 160.0 us.
+// NT: nontemporal stores. They are the faster ones alone (Q4_K 2000x2048 4.3
+// against 5.4 us), but the caller reads the tensor next, and a small one is then
+// still in the caches: with an fp32 matrix product of 64 rows behind it, 1024x1024
+// 15.7 against 13.2 us, 1024x2048 17.6 / 15.6, 2048x2048 25.6 / 25.4.
+template <int FMT, std::uint32_t PER, bool NT>
 __global__ __launch_bounds__(256) void dequant_kernel(const std::uint8_t* __restrict__ payload,
                                                       const std::uint8_t* __restrict__ meta, std::size_t blocks,
                                                       float* __restrict__ out) {
   const std::uint32_t lane = threadIdx.x & 63u;
-  const std::size_t b0 = (static_cast<std::size_t>(blockIdx.x) * 4u + (threadIdx.x >> 6)) * kDequantBlocks;
+  const std::size_t b0 = (static_cast<std::size_t>(blockIdx.x) * 4u + (threadIdx.x >> 6)) * PER;
   auto load = [&](std::size_t b) {
     return run4_load<FMT>(payload + b * rtxllm_format_payload_bytes(FMT),
                           meta != nullptr ? meta + b * rtxllm_format_meta_bytes(FMT) : nullptr, lane);
   };
   auto store = [&](std::size_t b, const float4& v) {
     const f32x4_any o = {v.x, v.y, v.z, v.w};
-    __builtin_nontemporal_store(o, reinterpret_cast<f32x4_any*>(out + b * 256u + 4u * lane));
+    f32x4_any* const dst = reinterpret_cast<f32x4_any*>(out + b * 256u + 4u * lane);
+    if constexpr (NT)
+      __builtin_nontemporal_store(o, dst);
+    else
+      *dst = o;
   };
-  if (b0 + kDequantBlocks <= blocks) {
-    Run4 r[kDequantBlocks];
+  if (b0 + PER <= blocks) {
+    Run4 r[PER];
 #pragma unroll
-    for (std::uint32_t j = 0; j < kDequantBlocks; ++j) r[j] = load(b0 + j);
+    for (std::uint32_t j = 0; j < PER; ++j) r[j] = load(b0 + j);
     __builtin_amdgcn_sched_barrier(0);  // every block's loads ahead of the first's arithmetic
 #pragma unroll
-    for (std::uint32_t j = 0; j < kDequantBlocks; ++j) store(b0 + j, run4_values<FMT>(r[j], lane));
+    for (std::uint32_t j = 0; j < PER; ++j) store(b0 + j, run4_values<FMT>(r[j], lane));
   } else {
     for (std::size_t b = b0; b < blocks; ++b) store(b, run4_values<FMT>(load(b), lane));
   }
@@ -123,13 +129,21 @@ hipError_t launch_units_pack(const std::uint8_t* raw, std::uint32_t rows, std::u
   return hipGetLastError();
 }
 
+constexpr std::size_t kDequantCached = 8192;  // blocks of 1 KB of output
+
 template <int FMT>
 hipError_t launch_dequant_fmt(const std::uint8_t* payload, const std::uint8_t* meta, std::uint32_t rows,
                               std::uint32_t cols, float* out, hipStream_t stream) {
   const std::size_t blocks = static_cast<std::size_t>(rows) * (cols / 256u);
-  constexpr std::size_t kPer = 4u * kDequantBlocks;  // blocks per workgroup
-  hipLaunchKernelGGL(dequant_kernel<FMT>, dim3(static_cast<unsigned>((blocks + kPer - 1u) / kPer)), dim3(256), 0,
-                     stream, payload, meta, blocks, out);
+  // Up to 8 MB of output: cached stores, and a block a wave: four leave CUs idle
+  // below 4 MB and gain little up to here (Q4_K 250x512 2.2 us with four, 2.0 with
+  // one; 500x2048 2.9 / 2.8; 1000x2048 3.3 / 3.6).
+  if (blocks <= kDequantCached)
+    hipLaunchKernelGGL((dequant_kernel<FMT, 1, false>), dim3(static_cast<unsigned>((blocks + 3u) / 4u)), dim3(256), 0,
+                       stream, payload, meta, blocks, out);
+  else
+    hipLaunchKernelGGL((dequant_kernel<FMT, 4, true>), dim3(static_cast<unsigned>((blocks + 15u) / 16u)), dim3(256), 0,
+                       stream, payload, meta, blocks, out);
   return hipGetLastError();
 }
 

@@ -62,10 +62,12 @@ def test_argmax_edges(orc, n, offset):
 
 
 @pytest.mark.parametrize("fmt", sorted(F.PAYLOAD_BYTES), ids=lambda f: F.NAMES[f])
-@pytest.mark.parametrize("rows,cols", [(1, 256), (3, 256), (5, 768), (7, 2304), (33, 4096)])
+@pytest.mark.parametrize("rows,cols", [(1, 256), (3, 256), (5, 768), (7, 2304), (33, 4096), (8192, 256),
+                                       (8195, 256), (2731, 768)])
 def test_dequant_edges_bit_exact(orc, fmt, rows, cols):
-    """Block counts around the kernel's 4 blocks a wave and 16 a workgroup, and an
-    output buffer off its 16-byte alignment; nothing past the end is written."""
+    """Block counts around the small outputs' one block a wave and the large ones'
+    four (from 8193 blocks on), and an output buffer off its 16-byte alignment;
+    nothing past the end is written."""
     pack = packs.make_pack(fmt, rows, cols, seed=900 + fmt)
     d = ops.DevicePack(pack)
     n = rows * cols
