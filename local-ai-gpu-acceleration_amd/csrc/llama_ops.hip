@@ -41,7 +41,7 @@ __device__ float block_sum256(float v, float* sh) {
 // weights are read ahead of the reduction. x, w and out 16-byte aligned, n % 4
 // == 0; in place allowed (a thread writes what it alone read). Against the
 // scalar two-pass kernel below (16 dependent loads, twice): one vector of 4096
-// 8.4 -> 2.4 us, 256 of them 11.5 -> 3.5 us.
+// 7.1 -> 2.3 us, 256 of them 8.0 -> 3.3 us.
 template <std::uint32_t T, std::uint32_t V>
 __global__ __launch_bounds__(T) void rmsnorm_w_vec_kernel(const float* x, const float* __restrict__ w, std::uint32_t n,
                                                           float eps, float* out) {
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(T) void rmsnorm_w_vec_kernel(const float* x, const 
   }
 }
 
-// The rest: unaligned pointers, n % 4 != 0, vectors over 16384 values.
+// The rest: unaligned pointers, n % 4 != 0, vectors under 128 or over 16384 values.
 __global__ __launch_bounds__(kOpThreads) void rmsnorm_w_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                                std::uint32_t n, float eps, float* __restrict__ out) {
   __shared__ float sh[kOpThreads / 64];
@@ -241,20 +241,20 @@ extern "C" hipError_t rtxllm_rmsnorm_w(const float* x, const float* weight, uint
     return hipErrorInvalidValue;
   // (a launch holds fewer than 2^32 threads: more than 2^22 - 1 vectors wider than
   // 4096 stay with the 256-thread kernel)
-  const bool vec = (n % 4u) == 0u && n <= 16384u && (n <= 4096u || count < (1u << 22)) &&
+  // (and vectors of less than half a wave's loads, which gain nothing: 16384 of 64
+  // 6.6 us scalar, 7.0 vector)
+  const bool vec = (n % 4u) == 0u && n >= 128u && n <= 16384u && (n <= 4096u || count < (1u << 22)) &&
                    ((reinterpret_cast<std::uintptr_t>(x) | reinterpret_cast<std::uintptr_t>(weight) |
                      reinterpret_cast<std::uintptr_t>(out)) % 16u) == 0u;
-  // Few vectors leave the chip idle and the one workgroup's latency is the time:
-  // 16 waves share a vector, one or a few loads each. From half a workgroup per
-  // CU on, four waves a vector keep more of them resident.
+  // Four waves a vector up to 4096 values: 16 waves, one load each, take longer to
+  // meet at the barrier also where one vector has the chip (one of 4096 2.35 us,
+  // four waves 2.24; 64 of 4096 2.61 / 2.50; 512 of 2048 3.54 / 3.35).
   if (!vec)
     hipLaunchKernelGGL(rmsnorm_w_kernel, dim3(count), dim3(kOpThreads), 0, stream, x, weight, n, eps, out);
   else if (n <= 1024u)
     hipLaunchKernelGGL((rmsnorm_w_vec_kernel<256, 1>), dim3(count), dim3(256), 0, stream, x, weight, n, eps, out);
-  else if (n <= 4096u && count >= 128u)
-    hipLaunchKernelGGL((rmsnorm_w_vec_kernel<256, 4>), dim3(count), dim3(256), 0, stream, x, weight, n, eps, out);
   else if (n <= 4096u)
-    hipLaunchKernelGGL((rmsnorm_w_vec_kernel<1024, 1>), dim3(count), dim3(1024), 0, stream, x, weight, n, eps, out);
+    hipLaunchKernelGGL((rmsnorm_w_vec_kernel<256, 4>), dim3(count), dim3(256), 0, stream, x, weight, n, eps, out);
   else
     hipLaunchKernelGGL((rmsnorm_w_vec_kernel<1024, 4>), dim3(count), dim3(1024), 0, stream, x, weight, n, eps, out);
   return hipGetLastError();

@@ -85,7 +85,7 @@ def test_dequant_edges_bit_exact(orc, fmt, rows, cols):
         assert np.all(got[:off] == 7.0) and np.all(got[off + n:] == 7.0)
 
 
-@pytest.mark.parametrize("n,count", [(1, 2), (6, 3), (256, 3), (1024, 1), (1028, 130), (4096, 127), (4096, 128),
+@pytest.mark.parametrize("n,count", [(1, 2), (6, 3), (124, 3), (128, 3), (256, 3), (1024, 1), (1028, 130), (4096, 127), (4096, 128),
                                      (4100, 2), (16384, 2), (16388, 2)])
 @pytest.mark.parametrize("offset", [0, 2])
 def test_rmsnorm_edges(n, count, offset):
