@@ -9,9 +9,6 @@
 namespace rtxllm {
 
 constexpr std::uint32_t kArgmaxThreads = 1024;
-// Rows of at most this many values run with short batches (argmax_row<2>):
-// all of such a row is one batch of two 16-byte loads a thread.
-constexpr std::uint32_t kArgmaxShort = 2u * 4u * kArgmaxThreads;
 
 // Maximum (a) and, with it, minimum over the workgroup's 16 waves; every thread
 // gets the result. The caller separates two uses of `sh` by a barrier.
@@ -32,17 +29,15 @@ __device__ __forceinline__ std::uint32_t argmax_block_reduce(std::uint32_t v, st
 // kArgmaxThreads workgroup calls it and gets the index. n >= 1; row has any
 // 4-byte alignment.
 //
-// One CU reads the whole row (a second launch or a cleared counter to share the
-// row among CUs costs more than the read), so the time is the row's latency:
-// a thread keeps U 16-byte loads in flight (128 KB per CU at U = 8) and only
-// the maximum of each batch of 4 U values is compared, the index being found
-// afterwards by reading the winning batch again. Against one 4-byte load and
-// compare at a time: the Q5_K LM-head launcher (128256 rows, token included)
-// 109.5 -> 74.8 us, a gather / norm / rotary / SiLU / argmax(128256) graph 45.3
-// -> 29.0 us, the 14336-row IQ2_S launcher 21.3 -> 18.7 us, a Q4_K stage of
-// 8192 rows 19.3 -> 17.9 us.
-template <std::uint32_t U>
+// One CU reads the whole row: the entry points have no scratch through which
+// several could share it. So the time is the row's latency: a thread keeps two
+// 16-byte loads in flight and only the maximum of each batch of eight values is
+// compared, the index being found afterwards by reading the winning batch again.
+// Against one 4-byte load and compare at a time: 8192 values 4.6 -> 2.8 us, 32768
+// 8.4 -> 3.6, 128256 23.6 -> 6.0. Eight loads a thread are slower at every length
+// (8193 values 4.6 us, two loads 2.8; 128256 7.6 / 6.0; 1000000 31.8 / 29.4).
 __device__ __forceinline__ std::uint32_t argmax_row(const float* __restrict__ row, std::uint32_t n) {
+  constexpr std::uint32_t U = 2;  // 16-byte loads of a batch
   __shared__ std::uint32_t sh[2][kArgmaxThreads / 64u];
   const std::uint32_t tid = threadIdx.x;
   // row = head (to the first 16-byte boundary), nv 16-byte vectors, tail

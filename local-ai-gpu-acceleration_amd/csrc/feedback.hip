@@ -115,13 +115,12 @@ hipError_t launch_feedback(const float* logits, const float* gate, float* cache,
 // ---- argmax ---------------------------------------------------------------
 
 // One workgroup per call (argmax.cuh: why, and the rules for ties and NaN).
-template <std::uint32_t U>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_token_kernel(const float* __restrict__ logits,
                                                                       std::uint32_t* token, std::uint32_t rows,
                                                                       int mode, std::uint32_t vocab,
                                                                       std::uint32_t offset) {
   const std::uint32_t before = (threadIdx.x == 0u && mode == 0) ? token[0] : 0u;  // read ahead of the scan
-  const std::uint32_t bi = argmax_row<U>(logits, rows);
+  const std::uint32_t bi = argmax_row(logits, rows);
   if (threadIdx.x == 0u) token[0] = mode == 0 ? (bi + before + 1u) % 32000u : (bi + offset) % vocab;
 }
 
@@ -129,12 +128,8 @@ __global__ __launch_bounds__(kArgmaxThreads) void argmax_token_kernel(const floa
 
 hipError_t launch_argmax_token(const float* logits, std::uint32_t* token, std::uint32_t rows, int mode,
                                std::uint32_t vocab, std::uint32_t offset, hipStream_t stream) {
-  if (rows <= kArgmaxShort)
-    hipLaunchKernelGGL(argmax_token_kernel<2>, dim3(1), dim3(kArgmaxThreads), 0, stream, logits, token, rows, mode,
-                       vocab, offset);
-  else
-    hipLaunchKernelGGL(argmax_token_kernel<8>, dim3(1), dim3(kArgmaxThreads), 0, stream, logits, token, rows, mode,
-                       vocab, offset);
+  hipLaunchKernelGGL(argmax_token_kernel, dim3(1), dim3(kArgmaxThreads), 0, stream, logits, token, rows, mode, vocab,
+                     offset);
   return hipGetLastError();
 }
 

@@ -196,10 +196,9 @@ __global__ __launch_bounds__(256) void embed_gather_q5k_kernel(const std::uint8_
 }
 
 // One workgroup per vector (argmax.cuh).
-template <std::uint32_t U>
 __global__ __launch_bounds__(kArgmaxThreads) void argmax_rows_kernel(const float* __restrict__ x, std::uint32_t n,
                                                                      std::uint32_t* __restrict__ index) {
-  const std::uint32_t i = argmax_row<U>(x + static_cast<std::size_t>(blockIdx.x) * n, n);
+  const std::uint32_t i = argmax_row(x + static_cast<std::size_t>(blockIdx.x) * n, n);
   if (threadIdx.x == 0u) index[blockIdx.x] = i;
 }
 
@@ -346,9 +345,6 @@ extern "C" hipError_t rtxllm_argmax(const float* x, uint32_t n, uint32_t count, 
                                     hipStream_t stream) {
   if (x == nullptr || index == nullptr || n == 0u || count == 0u || count > 65535u * 1024u)
     return hipErrorInvalidValue;
-  if (n <= kArgmaxShort)
-    hipLaunchKernelGGL(argmax_rows_kernel<2>, dim3(count), dim3(kArgmaxThreads), 0, stream, x, n, index);
-  else
-    hipLaunchKernelGGL(argmax_rows_kernel<8>, dim3(count), dim3(kArgmaxThreads), 0, stream, x, n, index);
+  hipLaunchKernelGGL(argmax_rows_kernel, dim3(count), dim3(kArgmaxThreads), 0, stream, x, n, index);
   return hipGetLastError();
 }
