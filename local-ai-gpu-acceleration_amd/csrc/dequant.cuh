@@ -1,7 +1,8 @@
 // Per-element dequant of the resident-pack layouts with the reference gate's
 // expression order (runtime/apps/mixed_sequence_benchmark_runner/main.cpp:
 // 1133-1259), compiled without FMA contraction: bit-exact with the CPU gate.
-// Used by the dequant entry point and the Q5_K embedding gather.
+// Used by the dequant entry point, the Q5_K embedding gather and the decode step's
+// embedding.
 #pragma once
 
 #include "mv.cuh"
@@ -9,20 +10,12 @@
 namespace rtxllm {
 
 #pragma clang fp contract(off)
-// Value v of a block, with the reference's expression order (main.cpp:1133-1259).
+// Value v of an IQ2_S or IQ3_S block (the unit layouts, whose bytes are gathered
+// first; every other layout expands four values a lane, below).
 template <int FMT>
-__device__ __forceinline__ float dequant_value(const std::uint8_t* p, const std::uint8_t* m, std::uint32_t v) {
-  if constexpr (FMT == RTXLLM_FMT_Q5K) {
-    const float d = f16_bits_to_f32(ld_u16(p));
-    const float dmin = f16_bits_to_f32(ld_u16(p + 2));
-    const std::uint32_t g = v >> 6, lane = v & 31u, high = (v & 63u) >= 32u;
-    std::uint32_t sc, mn;
-    scale_min_k4(static_cast<int>(2u * g + high), ld_u32(p + 4), ld_u32(p + 8), ld_u32(p + 12), sc, mn);
-    const std::uint32_t packed = p[48u + 32u * g + lane];
-    const std::uint32_t low = high ? (packed >> 4) : (packed & 15u);
-    const std::uint32_t quant = low + (((p[16u + lane] >> (2u * g + high)) & 1u) ? 16u : 0u);
-    return d * static_cast<float>(sc) * static_cast<float>(quant) - dmin * static_cast<float>(mn);
-  } else if constexpr (FMT == RTXLLM_FMT_IQ2S) {
+__device__ __forceinline__ float dequant_value(const std::uint8_t* p, std::uint32_t v) {
+  static_assert(FMT == RTXLLM_FMT_IQ2S || FMT == RTXLLM_FMT_IQ3S, "an IQ block");
+  if constexpr (FMT == RTXLLM_FMT_IQ2S) {
     const std::uint32_t ib32 = v >> 5, grp = (v & 31u) >> 3, lane = v & 7u;
     const float d = f16_bits_to_f32(ld_u16(p));
     const std::uint32_t go = ib32 * 4u + grp;
@@ -33,7 +26,7 @@ __device__ __forceinline__ float dequant_value(const std::uint8_t* p, const std:
     const float scale = d * (0.5f + static_cast<float>(nib)) * 0.25f;
     const bool neg = (p[34u + go] >> lane) & 1u;
     return scale * static_cast<float>(grid) * (neg ? -1.0f : 1.0f);
-  } else if constexpr (FMT == RTXLLM_FMT_IQ3S) {
+  } else {
     const std::uint32_t ib32 = v >> 5, grp = (v & 31u) >> 3, lane = v & 7u, pair = lane >> 2, gl = lane & 3u;
     const float d = f16_bits_to_f32(ld_u16(p));
     const std::uint32_t sel = ib32 * 8u + grp * 2u + pair;
@@ -45,28 +38,6 @@ __device__ __forceinline__ float dequant_value(const std::uint8_t* p, const std:
     const float scale = d * static_cast<float>(1u + 2u * nib);
     const bool neg = (p[74u + ib32 * 4u + grp] >> lane) & 1u;
     return scale * static_cast<float>(grid) * (neg ? -1.0f : 1.0f);
-  } else {
-    const std::uint32_t g = v >> 6, lane = v & 31u, high = (v & 63u) >= 32u, pair = 2u * g + high;
-    const std::uint8_t* qs = (FMT == RTXLLM_FMT_Q4K_RAW || FMT == RTXLLM_FMT_Q4K_RAW_PREDECODED) ? p + 16 : p;
-    const std::uint32_t packed = qs[32u * g + lane];
-    const float quant = static_cast<float>(high ? (packed >> 4) : (packed & 15u));
-    if constexpr (FMT == RTXLLM_FMT_Q4K_SPLIT_PREDECODED || FMT == RTXLLM_FMT_Q4K_RAW_PREDECODED) {
-      const float* pm = reinterpret_cast<const float*>(m) + 2u * pair;
-      return pm[0] * quant - pm[1];
-    } else if constexpr (FMT == RTXLLM_FMT_Q4K_SPLIT_HALF) {
-      return f16_bits_to_f32(ld_u16(m + 4u * pair)) * quant - f16_bits_to_f32(ld_u16(m + 4u * pair + 2u));
-    } else if constexpr (FMT == RTXLLM_FMT_Q4K_SPLIT_COMPACT) {
-      const float d = f16_bits_to_f32(ld_u16(m));
-      const float dmin = f16_bits_to_f32(ld_u16(m + 2));
-      return d * static_cast<float>(m[4u + pair]) * quant - dmin * static_cast<float>(m[12u + pair]);
-    } else {  // native head: split-native metadata or the raw block itself
-      const std::uint8_t* h = (FMT == RTXLLM_FMT_Q4K_RAW) ? p : m;
-      const float d = f16_bits_to_f32(ld_u16(h));
-      const float dmin = f16_bits_to_f32(ld_u16(h + 2));
-      std::uint32_t sc, mn;
-      scale_min_k4(static_cast<int>(pair), ld_u32(h + 4), ld_u32(h + 8), ld_u32(h + 12), sc, mn);
-      return d * static_cast<float>(sc) * quant - dmin * static_cast<float>(mn);
-    }
   }
 }
 
@@ -80,8 +51,8 @@ __device__ __forceinline__ void scale_min_select(std::uint32_t j, std::uint32_t 
 
 // Values 4 l .. 4 l + 3 of a block (lane l of the wave that holds the block) in
 // two steps, so that a wave can have several blocks' loads in flight: run4_load
-// reads the fields, run4_values expands them with dequant_value's expressions,
-// the same values bit for bit. The four values share the sub-block, its scale
+// reads the fields, run4_values expands them with the reference's expressions in
+// its order. The four values share the sub-block, its scale
 // (and min) and, in the IQ formats, the codebook word, so those are read and
 // decoded once; K-quant codes are one dword (blocks 4-byte aligned, or 2-byte in
 // the IQ formats, which read theirs as bytes).
@@ -170,7 +141,7 @@ __device__ __forceinline__ float4 run4_values(const Run4& r, std::uint32_t l) {
 // Values [16 t, 16 t + 16) of a Q5_K block (t in [0, 16)) from three aligned
 // 16-byte loads: the head (d, dmin, scales), the 16 qh bytes and the 16 qs
 // bytes the run uses (the run lies in one 32-value sub-block). Same values,
-// bit for bit, as dequant_value<Q5K> for each v in the run. The block must be
+// bit for bit, as run4_values<Q5K> over the run. The block must be
 // 16-byte aligned (176-byte blocks of a 16-byte aligned table are).
 __device__ __forceinline__ void dequant_q5k_run16(const std::uint8_t* blk, std::uint32_t t, float out[16]) {
   const std::uint32_t v0 = 16u * t, g = v0 >> 6, high = (v0 & 63u) >= 32u ? 1u : 0u, lane0 = v0 & 31u;

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void dequant_units_kernel(const std::uint8_t* 
   if (i < kRaw) blk[i] = payload[k2 ? iq2s_units_offset(b, i, nb) : iq3s_units_offset(b, i, nb)];
   __syncthreads();
   out[(b / bpr) * cols + (b % bpr) * 256u + i] =
-      dequant_value<k2 ? RTXLLM_FMT_IQ2S : RTXLLM_FMT_IQ3S>(blk, nullptr, i);
+      dequant_value<k2 ? RTXLLM_FMT_IQ2S : RTXLLM_FMT_IQ3S>(blk, i);
 }
 
 // One thread per block: GGUF IQ2_S / IQ3_S bytes -> the unit layout (IQ3_S:
