@@ -309,10 +309,8 @@ extern "C" hipError_t rtxllm_embed_gather_q5k(const uint8_t* table, uint32_t voc
 extern "C" size_t rtxllm_attn_decode_workspace(uint32_t n_heads, uint32_t n_kv_heads, uint32_t capacity,
                                                uint32_t count) {
   if (!group_ok(n_heads, n_kv_heads) || capacity == 0u || count == 0u) return 0u;
-  // the partials; the first term is room that an earlier staging of q needed and
-  // that callers' buffers have
-  return align256(static_cast<std::size_t>(count) * n_kv_heads * kQ16BytesPerKv) +
-         4u * static_cast<std::size_t>(count) * attention_partials_floats(n_heads, n_kv_heads, capacity);
+  // the partials of every chunk
+  return align256(4u * static_cast<std::size_t>(count) * attention_partials_floats(n_heads, n_kv_heads, capacity));
 }
 
 extern "C" hipError_t rtxllm_attn_decode_gqa_f16(const float* q, const uint16_t* k_cache, const uint16_t* v_cache,

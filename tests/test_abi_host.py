@@ -102,3 +102,12 @@ def test_synth_field_distributions():
     assert counts.min() > 0.95 * nib.size / 16
     x = packs.normal_f32(7, 200_000)
     assert abs(float(x.mean())) < 0.01 and abs(float(x.std()) - 1.0) < 0.01
+
+
+@pytest.mark.parametrize("heads,n_kv,capacity,count", [(1, 1, 64, 1), (32, 8, 4096, 8), (6, 3, 304, 3), (64, 8, 16384, 12)])
+def test_attention_workspace_holds_the_partials_alone(rlib, heads, n_kv, capacity, count):
+    """Per sequence, kv head and chunk of 128 positions the group's records of 128
+    sums, a maximum and a total; nothing for the queries, which need no staging."""
+    chunks = -(-capacity // 128)
+    partials = 4 * count * n_kv * chunks * (heads // n_kv) * (128 + 2)
+    assert rlib.rtxllm_attn_decode_workspace(heads, n_kv, capacity, count) == -(-partials // 256) * 256
