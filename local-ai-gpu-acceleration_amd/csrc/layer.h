@@ -65,16 +65,23 @@ hipError_t launch_attention(const void* q, const KvLayer& kv, std::uint32_t n_he
 // Per sequence partial-record floats of a launch over `span` positions (the
 // batch needs batch times as many).
 std::size_t attention_partials_floats(std::uint32_t n_heads, std::uint32_t n_kv, std::uint32_t span);
-// The same for `batch` sequences: sequence s has q16 n_kv * kQ16BytesPerKv
-// bytes on (q_f32: q is instead the fp32 queries [batch][n_heads][kHeadDim] of
-// any 4-byte alignment, before the 1 / sqrt(head_dim)), block-table row s (table_stride entries, >= capacity /
-// page_size), position pos[s], and writes att[s]; xq_att must be null when
-// batch > 1. x16_att (batch <= 8, xq_att null): att of every sequence is also
-// staged there for the batched o projection (the launch_stage_batch rule;
-// sequences >= batch zero), in the same launch as the combine.
-hipError_t launch_attention_batch(const void* q, bool q_f32, const KvLayer& kv, std::uint32_t n_heads, const std::uint32_t* pos,
-                                  std::uint32_t span, std::uint32_t batch, std::uint32_t table_stride,
-                                  float* partials, float* att, void* xq_att, void* x16_att, hipStream_t stream);
+// The queries of a launch, one of the two: staged operands (n_kv * kQ16BytesPerKv
+// bytes a sequence, 16-byte aligned), or fp32 [batch][n_heads][kHeadDim] of any
+// 4-byte alignment, before the 1 / sqrt(head_dim).
+struct AttnQuery {
+  const void* q16;
+  const float* f32;
+};
+// The same for `batch` sequences: sequence s has the s-th part of q, block-table
+// row s (table_stride entries, >= capacity / page_size), position pos[s], and
+// writes att[s]; xq_att must be null when batch > 1. x16_att (batch <= 8, xq_att
+// null): att of every sequence is also staged there for the batched o projection
+// (the launch_stage_batch rule; sequences >= batch zero), in the same launch as the
+// combine.
+hipError_t launch_attention_batch(const AttnQuery& q, const KvLayer& kv, std::uint32_t n_heads,
+                                  const std::uint32_t* pos, std::uint32_t span, std::uint32_t batch,
+                                  std::uint32_t table_stride, float* partials, float* att, void* xq_att, void* x16_att,
+                                  hipStream_t stream);
 
 // h += W x (rows % 16 == 0), x either the staged input xq_in or the fp32 x_in
 // (staged by each wave itself; exactly one of the two non-null); then xq_next =

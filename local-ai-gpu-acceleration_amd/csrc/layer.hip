@@ -330,7 +330,7 @@ constexpr std::uint32_t kMaxGroup = 8;
 // place of a staging launch and its buffer: eight sequences of up to 4096
 // positions 23.0 -> 21.9 us.
 template <int GROUP, bool EARLY_V, bool QF32 = false>
-__global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const void* __restrict__ q_in, KvLayer kv,
+__global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const std::conditional_t<QF32, float, _Float16>* __restrict__ q, KvLayer kv,
                                                                        const std::uint32_t* __restrict__ pos_ptr,
                                                                        std::uint32_t nchunks,
                                                                        float* __restrict__ partials,
@@ -361,11 +361,11 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const voi
   typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
   f32x4_any qf;
   if constexpr (QF32) {
-    const float* qr = static_cast<const float*>(q_in) + static_cast<std::size_t>(seq) * q_stride + g * (GROUP * kHeadDim);
+    const float* qr = q + static_cast<std::size_t>(seq) * q_stride + g * (GROUP * kHeadDim);
     qf = *reinterpret_cast<const f32x4_any*>(qr + 4u * (threadIdx.x % kQThreads));  // past them: read again, not used
   } else {
-    const _Float16* q = static_cast<const _Float16*>(q_in) + static_cast<std::size_t>(seq) * q_stride;
-    const uint4* qr = reinterpret_cast<const uint4*>(q + static_cast<std::size_t>(g) * kQ16PerKv) + lane;
+    const uint4* qr = reinterpret_cast<const uint4*>(q + static_cast<std::size_t>(seq) * q_stride +
+                                                     static_cast<std::size_t>(g) * kQ16PerKv) + lane;
 #pragma unroll
     for (int j = 0; j < 4; ++j) qb[j] = qr[64 * j];
   }
@@ -753,12 +753,13 @@ std::size_t attention_partials_floats(std::uint32_t n_heads, std::uint32_t n_kv,
   return static_cast<std::size_t>(n_kv) * nchunks * (n_heads / n_kv) * (kHeadDim + 2u);
 }
 
-hipError_t launch_attention_batch(const void* q, bool q_f32, const KvLayer& kv, std::uint32_t n_heads, const std::uint32_t* pos,
-                                  std::uint32_t span, std::uint32_t batch, std::uint32_t table_stride,
-                                  float* partials, float* att, void* xq_att, void* x16_att, hipStream_t stream) {
+hipError_t launch_attention_batch(const AttnQuery& q, const KvLayer& kv, std::uint32_t n_heads,
+                                  const std::uint32_t* pos, std::uint32_t span, std::uint32_t batch,
+                                  std::uint32_t table_stride, float* partials, float* att, void* xq_att, void* x16_att,
+                                  hipStream_t stream) {
   if (kv.n_kv == 0u || n_heads % kv.n_kv != 0u || n_heads / kv.n_kv > kMaxGroup || kv.capacity == 0u ||
       span == 0u || span > kv.capacity || kv.page_size == 0u || kv.capacity % kv.page_size != 0u || batch == 0u ||
-      batch > 65535u || (batch > 1u && (xq_att != nullptr || table_stride < kv.capacity / kv.page_size)))
+      batch > 65535u || (q.q16 == nullptr) == (q.f32 == nullptr) || (batch > 1u && (xq_att != nullptr || table_stride < kv.capacity / kv.page_size)))
     return hipErrorInvalidValue;
   if (x16_att != nullptr && (xq_att != nullptr || batch > kBatchMax || (n_heads * kHeadDim) % 256u != 0u))
     return hipErrorInvalidValue;
@@ -769,21 +770,22 @@ hipError_t launch_attention_batch(const void* q, bool q_f32, const KvLayer& kv, 
   const std::size_t part = attention_partials_floats(n_heads, kv.n_kv, span);
   if (part > 0xFFFFFFFFull) return hipErrorInvalidValue;
   const std::uint32_t part_stride = static_cast<std::uint32_t>(part);
-  const std::uint32_t q_stride = q_f32 ? n_heads * kHeadDim : kv.n_kv * kQ16PerKv;
+  const std::uint32_t q_stride = q.f32 != nullptr ? n_heads * kHeadDim : kv.n_kv * kQ16PerKv;
   const dim3 grid(nchunks, kv.n_kv, batch), block(64 * kAttnWaves);
-#define RTXLLM_ATTN_LAUNCH(G, EARLY_V, QF32)                                                                       \
-  hipLaunchKernelGGL((attn_partial_kernel<G, EARLY_V, QF32>), grid, block, 0, stream, q, kv, pos, nchunks, partials, \
+  const auto* const q16 = static_cast<const _Float16*>(q.q16);
+#define RTXLLM_ATTN_LAUNCH(G, EARLY_V, QF32, Q)                                                                    \
+  hipLaunchKernelGGL((attn_partial_kernel<G, EARLY_V, QF32>), grid, block, 0, stream, Q, kv, pos, nchunks, partials, \
                      q_stride, table_stride, part_stride)
 #define RTXLLM_ATTN_CASE(G)                            \
   case G:                                              \
-    if (q_f32 && batch > 1u)                           \
-      RTXLLM_ATTN_LAUNCH(G, true, true);               \
-    else if (q_f32)                                    \
-      RTXLLM_ATTN_LAUNCH(G, false, true);              \
+    if (q.f32 != nullptr && batch > 1u)                \
+      RTXLLM_ATTN_LAUNCH(G, true, true, q.f32);        \
+    else if (q.f32 != nullptr)                         \
+      RTXLLM_ATTN_LAUNCH(G, false, true, q.f32);       \
     else if (batch > 1u)                               \
-      RTXLLM_ATTN_LAUNCH(G, true, false);              \
+      RTXLLM_ATTN_LAUNCH(G, true, false, q16);         \
     else                                               \
-      RTXLLM_ATTN_LAUNCH(G, false, false);             \
+      RTXLLM_ATTN_LAUNCH(G, false, false, q16);        \
     break;
   switch (group) {
     RTXLLM_ATTN_CASE(1)
@@ -810,7 +812,7 @@ hipError_t launch_attention_batch(const void* q, bool q_f32, const KvLayer& kv, 
 hipError_t launch_attention(const void* q, const KvLayer& kv, std::uint32_t n_heads, const std::uint32_t* pos,
                             std::uint32_t span, float* partials, float* att, void* xq_att, hipStream_t stream) {
   if (xq_att == nullptr) return hipErrorInvalidValue;
-  return launch_attention_batch(q, false, kv, n_heads, pos, span, 1u, 0u, partials, att, xq_att, nullptr, stream);
+  return launch_attention_batch(AttnQuery{q, nullptr}, kv, n_heads, pos, span, 1u, 0u, partials, att, xq_att, nullptr, stream);
 }
 
 hipError_t launch_residual(int fmt, const std::uint8_t* payload, const std::uint8_t* meta, std::uint32_t rows,

@@ -335,8 +335,8 @@ extern "C" hipError_t rtxllm_attn_decode_gqa_f16(const float* q, const uint16_t*
   kv.page_size = page_size;
   kv.n_kv = n_kv_heads;
   kv.capacity = capacity;
-  return launch_attention_batch(q, true, kv, n_heads, pos, capacity, count, table_stride, partials, out, nullptr, nullptr,
-                                stream);
+  return launch_attention_batch(AttnQuery{nullptr, q}, kv, n_heads, pos, capacity, count, table_stride, partials, out,
+                                nullptr, nullptr, stream);
 }
 
 extern "C" hipError_t rtxllm_argmax(const float* x, uint32_t n, uint32_t count, uint32_t* index,

@@ -726,8 +726,8 @@ hipError_t launch_stage_batch(rtxllm_llama* m, std::uint32_t l, int stage, bool 
                                          m->pages_per_seq, stream);
     }
     case kAttention: {
-      return rtxllm::launch_attention_batch(m->arena.arena_ptr("q"), false, kv_layer(m, l), c.n_heads, pos, m->span, B,
-                                            m->pages_per_seq, region<float>(m, "attn_partials"),
+      return rtxllm::launch_attention_batch({m->arena.arena_ptr("q"), nullptr}, kv_layer(m, l), c.n_heads, pos, m->span,
+                                            B, m->pages_per_seq, region<float>(m, "attn_partials"),
                                             region<float>(m, "att"), nullptr, x16, stream);
     }
     case kO: {
