@@ -25,7 +25,6 @@ namespace {
 // block, the 65 of an 8B batch-8 step take 30 us less (3012 -> 2982 us).
 
 constexpr std::uint32_t kStageThreads = 64;
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));   // x of any 4-byte alignment
 typedef _Float16 half4 __attribute__((ext_vector_type(4), aligned(2)));
 
 // Sum of a block's 256 values, lane l holding values 4 l .. 4 l + 3, as a fixed

@@ -13,6 +13,10 @@ namespace rtxllm {
 
 constexpr int kWave = 64;
 
+// Four floats loaded or stored at once at any 4-byte alignment (a caller's buffer;
+// gfx950 takes unaligned 16-byte vectors).
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+
 // IEEE binary16 -> fp32 with the reference's NaN rule (any NaN becomes the
 // canonical +quiet NaN, decode_kernels.cu:1665-1676). The hardware conversion is
 // exact for every finite and infinite input.

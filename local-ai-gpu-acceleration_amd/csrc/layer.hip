@@ -358,7 +358,6 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attn_partial_kernel(const std
   uint4 qb[4];
   constexpr std::uint32_t kQThreads = GROUP * kHeadDim / 4u;  // QF32: four dims a thread
   __shared__ __align__(16) _Float16 q16s[QF32 ? kQ16PerKv : 8u];
-  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
   f32x4_any qf;
   if constexpr (QF32) {
     const float* qr = q + static_cast<std::size_t>(seq) * q_stride + g * (GROUP * kHeadDim);

@@ -180,7 +180,6 @@ __global__ __launch_bounds__(256) void embed_gather_q5k_kernel(const std::uint8_
                                                                std::uint32_t vocab, std::uint32_t cols,
                                                                const std::uint32_t* __restrict__ tokens,
                                                                float* __restrict__ out) {
-  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
   const std::uint32_t b = 4u * blockIdx.x + (threadIdx.x >> 6), t = blockIdx.y, bpr = cols / 256u;
   const std::uint32_t lane = threadIdx.x & 63u;
   if (b >= bpr) return;

@@ -41,10 +41,6 @@ bool pointers_ok(int fmt, const void* payload, const void* meta, const void* x, 
 // ---- bit-exact dequant -----------------------------------------------------
 
 
-// Four fp32 outputs stored at once; the caller's buffer may have any 4-byte
-// alignment (gfx950 stores unaligned 16-byte vectors).
-typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
-
 // A wave expands PER consecutive blocks (out is the blocks in order: 256 values
 // each), lane l four values of each: 1 KB of whole lines per store. The kernel is
 // bound by its writes (fp32 out is 7 to 12 times the pack's bytes). Q4_K 14336 x

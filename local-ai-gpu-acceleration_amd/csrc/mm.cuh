@@ -292,7 +292,7 @@ __device__ __forceinline__ void mm_block_scale(const MmRaw& r, float& d, float& 
 // of the launch (TCP_TOTAL_CACHE_ACCESSES 52.7k per CU in 57k cycles), the VALU
 // 46 %, the LDS 26 %. Where a workgroup's row segment is a whole number of 16-byte
 // pieces (mm_lds_fits), it therefore copies each tile's 16 row segments to LDS
-// with whole-line loads, kMmPieces 16-byte pieces a thread, and the lanes read
+// with whole-line loads, mm_pieces 16-byte pieces a thread, and the lanes read
 // their fields there. A row segment's image: its payload blocks, then (Q4_K
 // split-native) its heads, then 16 bytes of padding that spread the rows over the
 // banks.
@@ -312,11 +312,13 @@ constexpr std::uint32_t mm_head_pieces() {
   return FmtBytes<FMT>::meta > 0u ? (kPanelBlocks * FmtBytes<FMT>::meta + 63u) / 64u : 0u;
 }
 // Whether workgroups of `waves` panels (one: of a single tile each) take the LDS
-// path: their segments start and end on 16-byte pieces of the stream (IQ blocks of
-// 82 and 110 bytes: 16 of them), and they fill a CU as one workgroup, as the field
-// loads' kernel does (smaller workgroups rely on several a CU, which the tiles'
-// LDS would not hold). Within that the faster one is taken, us of the field loads
-// / of LDS, batch 8, cold weights:
+// path. Their segments have to start and end on 16-byte pieces of the stream, for
+// IQ blocks of 82 and 110 bytes groups of eight of them; it is built for eight
+// panels (K-quants: also seven), whose workgroup fills a CU with either path. Fewer
+// panels read fields: the image is sized for eight whatever the workgroup has, so
+// several would not share a CU, and a smaller image has not been measured. Within
+// that the faster one is taken, us of the field loads / of LDS, batch 8, cold
+// weights:
 //  * IQ: IQ2_S 28672x4096 23.5 / 20.0, 4096x4096 8.1 / 6.3; IQ3_S 27.6 / 23.6, 8.8
 //    / 6.7; with self-staging 14336x4096 19.4 / 17.6 and 21.7 / 19.8;
 //  * K-quants, whose field loads are whole 16 bytes a lane, gain less and lose the
@@ -770,7 +772,6 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
 // (batch 8, Q4_K 4096 x 14336, four groups: 17.9 -> 17.2 us with the matvec).
 __global__ __launch_bounds__(64) void mm_reduce_kernel(const float* __restrict__ partial, std::uint32_t groups,
                                                        std::uint32_t n, float* __restrict__ y) {
-  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
   const std::uint32_t i = 4u * (blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= n) return;
   if (n - i < 4u) {

@@ -918,7 +918,6 @@ __global__ __launch_bounds__(64 * EpiWaves<Epi>::value) void mv_kernel(QTensor w
   f32x16 xf0[UPL], xf1[UPL];
   // SHARE: quads of four values tid, tid + threads, ...: the first two a thread
   // here (all of them, up to 8 values a thread), any others below
-  typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
   const std::uint32_t quads = w.cols / 4u;
   f32x4_any xq4[SHARE ? 2 : 1];
   if constexpr (SHARE) {
@@ -978,8 +977,8 @@ __global__ __launch_bounds__(64 * EpiWaves<Epi>::value) void mv_kernel(QTensor w
       xg_quant(xf0[i], x0[i]);
       xg_quant(xf1[i], x1[i]);
     }
-    tl_stamp(kTlR >= 0 ? kTlSelfStaged : -1, tl_slot / 2u);
   }
+  if constexpr (SELF) tl_stamp(kTlR >= 0 ? kTlSelfStaged : -1, tl_slot / 2u);
   if constexpr (kPair) {
     ready[wave] = 0u;
     taken[wave] = 0u;

@@ -152,19 +152,13 @@ struct XQuad {
   std::uint32_t h, m, l;
   float s, sum;
 };
-__device__ __forceinline__ std::uint32_t xq_quad_dpp1(std::uint32_t v) {
-  return static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0xB1, 0xF, 0xF, false));
-}
-__device__ __forceinline__ std::uint32_t xq_quad_dpp2(std::uint32_t v) {
-  return static_cast<std::uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x4E, 0xF, 0xF, false));
-}
 __device__ __forceinline__ XQuad quant4(const float v[4]) {
   float m = fmaxf(fmaxf(fmaxf(0.0f, fabsf(v[0])), fmaxf(fabsf(v[1]), fabsf(v[2]))), fabsf(v[3]));
   std::uint32_t nan = __builtin_isunordered(v[0], v[1]) || __builtin_isunordered(v[2], v[3]) ? 1u : 0u;
-  m = fmaxf(m, __uint_as_float(xq_quad_dpp1(__float_as_uint(m))));
-  m = fmaxf(m, __uint_as_float(xq_quad_dpp2(__float_as_uint(m))));
-  nan |= xq_quad_dpp1(nan);
-  nan |= xq_quad_dpp2(nan);
+  m = fmaxf(m, __uint_as_float(dpp_bits<0xB1>(__float_as_uint(m))));
+  m = fmaxf(m, __uint_as_float(dpp_bits<0x4E>(__float_as_uint(m))));
+  nan |= dpp_bits<0xB1>(nan);
+  nan |= dpp_bits<0x4E>(nan);
   const XScale sc = xq_scale(m, nan != 0u);
   std::uint32_t Y[4], total = 0u;
 #pragma unroll
@@ -173,8 +167,8 @@ __device__ __forceinline__ XQuad quant4(const float v[4]) {
     total += static_cast<std::uint32_t>(X);
     Y[b] = static_cast<std::uint32_t>(X + kXQBias);
   }
-  total += xq_quad_dpp1(total);
-  total += xq_quad_dpp2(total);
+  total += dpp_bits<0xB1>(total);
+  total += dpp_bits<0x4E>(total);
   const std::uint32_t p01 = __builtin_amdgcn_perm(Y[1], Y[0], 0x05010400u);  // as in quant16
   const std::uint32_t p23 = __builtin_amdgcn_perm(Y[3], Y[2], 0x05010400u);
   const std::uint32_t q01 = __builtin_amdgcn_perm(Y[1], Y[0], 0x06020602u);
