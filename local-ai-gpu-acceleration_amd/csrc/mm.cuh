@@ -685,7 +685,7 @@ __global__ __launch_bounds__(64 * kMaxPanels) void mm_kernel(QTensor w, const vo
         // whose LDS serves the codebook lookups, it cost gate_up 4 %, Q4_K
         // 28672x4096 1 % and self-staging 2 %). A single panel has nothing to wait
         // for: the eight clamped reads cost it 3 to 6 % (4096x512: 3.9 -> 4.2 us)
-        if (nw == 1u) {
+        if (!LDSW && nw == 1u) {  // through LDS there are seven or eight
           v = red[round & 1u][0][e];
         } else {
           float r[kMaxPanels];
