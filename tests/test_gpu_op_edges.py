@@ -26,6 +26,28 @@ def at_offset(a: np.ndarray, floats: int) -> torch.Tensor:
     return view
 
 
+def row_slice(pack: packs.Pack, first: int, rows: int) -> packs.Pack:
+    """Rows [first, first + rows) of a row-major pack as a pack of its own."""
+    nb = pack.cols // 256
+
+    def part(a, width):
+        return np.ascontiguousarray(a.reshape(-1)[first * nb * width:(first + rows) * nb * width])
+
+    return packs.Pack(pack.fmt, rows, pack.cols, part(pack.payload, F.PAYLOAD_BYTES[pack.fmt]),
+                      None if pack.meta is None else part(pack.meta, F.META_BYTES[pack.fmt]))
+
+
+def matvec_batch_f32(w: ops.DevicePack, x: torch.Tensor) -> np.ndarray:
+    """rtxllm_matvec_batch_f32 of x [batch][cols]."""
+    batch = x.shape[0]
+    need = int(lib().rtxllm_matvec_batch_workspace(w.fmt, w.rows, w.cols))
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda:0")
+    y = torch.empty((batch, w.rows), dtype=torch.float32, device="cuda:0")
+    assert lib().rtxllm_matvec_batch_f32(w.fmt, P(w.payload), P(w.meta), P(x), P(y), w.rows, w.cols, batch, P(ws), need,
+                                         ops.stream()) == 0
+    return y.cpu().numpy()
+
+
 @pytest.mark.parametrize("n", [1, 2, 3, 4, 5, 7, 4095, 4096, 8191, 8192, 8193, 32767, 32773, 128259])
 @pytest.mark.parametrize("offset", [0, 1, 3])
 def test_argmax_edges(orc, n, offset):
@@ -162,19 +184,22 @@ def test_silu_mul_edges(orc, n, offset):
 
 
 @pytest.mark.parametrize("fmt", [F.Q4K_RAW, F.Q4K_SPLIT_NATIVE, F.Q5K, F.IQ2S, F.IQ3S], ids=lambda f: F.NAMES[f])
-@pytest.mark.parametrize("cols", [512, 4096])
+@pytest.mark.parametrize("cols", [512, 2048, 3072, 4096])
 def test_batch_single_tile_equals_many_tiles(fmt, cols):
-    """The single-tile kernel (few rows, every tile resident) and the ring over
-    many tiles give a row the same bits; rows % 16 != 0 in both."""
+    """The single-tile kernels (few rows, every tile resident; by format and panels
+    also the ring over one tile) and the ring over many tiles give a row the same
+    bits, staged and self-staging; rows % 16 != 0 in both."""
     rows, few, batch = 70001 if cols == 512 else 16393, 71, 5
     pack = packs.make_pack(fmt, rows, cols, seed=40 + fmt)
-    blocks = few * (cols // 256)
-    head = packs.Pack(fmt, few, cols, pack.payload[:blocks * F.PAYLOAD_BYTES[fmt]],
-                      None if pack.meta is None else pack.meta[:blocks * F.META_BYTES[fmt]])
-    x16 = ops.stage_batch(ops.to_dev(packs.normal_f32(9, batch * cols).reshape(batch, cols)))
+    xd = ops.to_dev(packs.normal_f32(9, batch * cols).reshape(batch, cols))
+    x16 = ops.stage_batch(xd)
     many = ops.matvec_batch(ops.DevicePack(pack), x16, batch).cpu().numpy()
-    one = ops.matvec_batch(ops.DevicePack(head), x16, batch).cpu().numpy()
-    assert np.array_equal(many[:, :few].view(np.uint32), one.view(np.uint32))
+    # the first rows (round 0 of the first workgroups), some of a middle round and
+    # the last ones with the ragged tile
+    for first in (0, rows // 2, rows - few):
+        w = ops.DevicePack(row_slice(pack, first, few))
+        for one in (ops.matvec_batch(w, x16, batch).cpu().numpy(), matvec_batch_f32(w, xd)):
+            assert np.array_equal(many[:, first:first + few].view(np.uint32), one.view(np.uint32)), first
 
 
 @pytest.mark.parametrize("heads,n_kv", [(1, 1), (6, 3), (4, 1), (16, 2)])
@@ -258,26 +283,51 @@ def test_matvec_shared_staging_equals_staged_input(fmt, rows, cols):
 
 
 @pytest.mark.parametrize("fmt", [F.Q4K_RAW, F.Q4K_SPLIT_NATIVE, F.Q5K, F.IQ2S, F.IQ3S], ids=lambda f: F.NAMES[f])
-@pytest.mark.parametrize("rows", [1, 100, 16400])
+@pytest.mark.parametrize("rows", [1, 100, 6001, 16393])
 @pytest.mark.parametrize("wide", [3584, 4096, 8192])
 def test_batch_weights_through_lds_equal_field_loads(fmt, rows, wide):
     """Workgroups of seven or eight panels copy their weights through LDS (or, by the
-    rule, do not), smaller ones read fields: with x zero past the first 2048
-    columns the wide matrix gives the bits of its left 2048 columns."""
-    batch, left = 3, 2048
+    rule, do not), smaller ones read fields: with x zero but for a window of 2048
+    columns the wide matrix gives the bits of those columns alone. The windows
+    cover every panel of the workgroup and, at 8192 columns, both panel groups.
+    Rows of one tile, several, more tiles than CUs (376: single tiles, two a CU)
+    and many rounds, the last tile ragged. Self-staging gives the same bits."""
+    batch, part_cols = 3, 2048
     pack = packs.make_pack(fmt, rows, wide, seed=60 + fmt)
+    w = ops.DevicePack(pack)
     pb, mb, nb = F.PAYLOAD_BYTES[fmt], F.META_BYTES.get(fmt, 0), wide // 256
 
-    def part(a, width):
-        return np.ascontiguousarray(a.reshape(rows, nb, width)[:, :left // 256]).reshape(-1)
+    def part(a, width, first):
+        return np.ascontiguousarray(a.reshape(rows, nb, width)[:, first // 256:(first + part_cols) // 256]).reshape(-1)
 
-    narrow = packs.Pack(fmt, rows, left, part(pack.payload, pb), None if pack.meta is None else part(pack.meta, mb))
-    x = np.zeros((batch, wide), np.float32)
-    x[:, :left] = packs.normal_f32(5, batch * left).reshape(batch, left)
-    y = ops.matvec_batch(ops.DevicePack(pack), ops.stage_batch(ops.to_dev(x)), batch).cpu().numpy()
-    xs = np.ascontiguousarray(x[:, :left])
-    ref = ops.matvec_batch(ops.DevicePack(narrow), ops.stage_batch(ops.to_dev(xs)), batch).cpu().numpy()
-    assert np.array_equal(y, ref)
+    for first in sorted({*range(0, wide - part_cols + 1, part_cols), wide - part_cols}):
+        narrow = packs.Pack(fmt, rows, part_cols, part(pack.payload, pb, first),
+                            None if pack.meta is None else part(pack.meta, mb, first))
+        xs = packs.normal_f32(5, batch * part_cols).reshape(batch, part_cols)
+        x = np.zeros((batch, wide), np.float32)
+        x[:, first:first + part_cols] = xs
+        xd = ops.to_dev(x)
+        ref = ops.matvec_batch(ops.DevicePack(narrow), ops.stage_batch(ops.to_dev(xs)), batch).cpu().numpy()
+        assert np.array_equal(ops.matvec_batch(w, ops.stage_batch(xd), batch).cpu().numpy(), ref), first
+        assert np.array_equal(matvec_batch_f32(w, xd), ref), first
+
+
+@pytest.mark.parametrize("fmt", [F.IQ2S, F.IQ3S], ids=lambda f: F.NAMES[f])
+@pytest.mark.parametrize("rows", [71, 16393])
+def test_batch_weights_through_lds_two_byte_payload(fmt, rows):
+    """An IQ payload 2 bytes past a 16-byte boundary, the least its entry points
+    take, gives the bits of the aligned one, staged and self-staging."""
+    cols, batch = 4096, 3
+    w = ops.DevicePack(packs.make_pack(fmt, rows, cols, seed=90 + fmt))
+    xd = ops.to_dev(packs.normal_f32(6, batch * cols).reshape(batch, cols))
+    ref = ops.matvec_batch(w, ops.stage_batch(xd), batch).cpu().numpy()
+    big = torch.zeros(w.payload.numel() + 16, dtype=torch.uint8, device="cuda:0")
+    moved = big[2:2 + w.payload.numel()]
+    moved.copy_(w.payload.reshape(-1))
+    w.payload = moved
+    assert w.payload.data_ptr() % 16 == 2
+    assert np.array_equal(ops.matvec_batch(w, ops.stage_batch(xd), batch).cpu().numpy(), ref)
+    assert np.array_equal(matvec_batch_f32(w, xd), ref)
 
 
 @pytest.mark.parametrize("rows,batch", [(1, 1), (3, 1), (5, 3), (64, 8), (1023, 7)])
@@ -292,3 +342,13 @@ def test_batch_panel_groups_are_added(orc, rows, batch, cols):
         ref = orc.matvec_f32(F.Q4K_SPLIT_NATIVE, pack.payload, pack.meta, xs[s], rows, cols, 8)
         # the fp32 sequential oracle's own error at these widths
         assert float(np.max(np.abs(y[s] - ref))) <= 1e-4 * float(np.max(np.abs(ref)))
+    # x zero outside a group's columns leaves that group's partial alone: the bits
+    # of y are those partials added in group order
+    panels = cols // 512
+    width = 512 * max(d for d in range(1, 9) if panels % d == 0)
+    total = np.zeros_like(y)
+    for first in range(0, cols, width):
+        xg = np.zeros_like(xs)
+        xg[:, first:first + width] = xs[:, first:first + width]
+        total += ops.matvec_batch(ops.DevicePack(pack), ops.stage_batch(ops.to_dev(xg)), batch).cpu().numpy()
+    assert np.array_equal(y, total)
