@@ -155,9 +155,9 @@ __global__ __launch_bounds__(kOpThreads) void silu_mul_kernel(const float* __res
 }
 
 // Four values a thread where the three pointers are 16-byte aligned; the last
-// n % 4 values one each by the first threads past the vectors. 14336 values 4.6 -> 2.1 us
-// against one value a thread; 256 x 14336 9.0 -> 8.0 us (44 MB: 5.5 TB/s, at the
-// copy rate).
+// n % 4 values one each by the first threads past the vectors. 14336 values 4.6 ->
+// 2.1 us against one value a thread; 256 x 14336 9.0 -> 8.0 us (44 MB: 5.5 TB/s;
+// a 1 GiB copy reaches 5.15).
 __global__ __launch_bounds__(kOpThreads) void silu_mul_vec_kernel(const float* gate, const float* up, std::size_t n,
                                                                   float* out) {
   const std::size_t i = static_cast<std::size_t>(blockIdx.x) * kOpThreads + threadIdx.x, n4 = n / 4u;

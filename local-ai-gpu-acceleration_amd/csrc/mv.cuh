@@ -795,7 +795,7 @@ __device__ __forceinline__ void pair_publish(std::uint32_t* counter, std::uint32
 // workgroup stages x once, four values a thread, into LDS, and every row group
 // reads its digits there. Otherwise each wave converts its own columns, 2 x 16
 // values a lane (~350 VALU), which for a launch of one or two tiles a wave is
-// as much work as a tile: IQ2_S 14336 x 4096 from fp32 x 14.1 -> 9.8 us (the
+// as much work as a tile: IQ2_S 14336 x 4096 from fp32 x 14.6 -> 10.8 us (the
 // rule and its figures: mv_share_groups).
 template <int FMT, int UPL, int TILE, bool SELF, class Epi, bool SHARE = false>
 __global__ __launch_bounds__(64 * EpiWaves<Epi>::value) void mv_kernel(QTensor w, XSrc xs, std::uint32_t rows,
